@@ -197,6 +197,10 @@ bool mtile_supported(int type);
 int launch_mtile(int type, const uint8_t* w, long long row_bytes, const Act& act, YOut y,
                  long long ldy, int m_rows, int n_rows, hipStream_t stream);
 
+// Prefill on 32 x 32 tiles (mxa_ptile.hip), any m_rows: Q4_K, Q6_K, Q8_0 on Q8_K activations.
+int launch_ptile(int type, const uint8_t* w, long long row_bytes, const Act& act, YOut y, long long ldy,
+                 int m_rows, int n_rows, hipStream_t stream);
+
 // Grouped MoE projection (mxa_mtile.hip): expert e of n_experts multiplies rows
 // [offsets[e], offsets[e + 1]) of the total_rows Q8_K activation rows in `act` (a device array of
 // n_experts + 1 ascending offsets; at most max_rows rows per expert) by its packed weight

@@ -1,4 +1,5 @@
-// Matrix-core matmul for M > 4 activation rows (batched decode and prefill), Q4_K / Q6_K / Q8_0.
+// Matrix-core matmul on 16 x 16 tiles, Q4_K / Q6_K / Q8_0: up to 64 activation rows, and the grouped
+// MoE forms (more rows: mxa_ptile.hip).
 //
 // Tiling. A workgroup of WAVES waves owns 16 * NT consecutive weight rows per wave and 16 * MT
 // activation rows; grid.y walks the activation rows, so a weight block is read once per 16 * MT
@@ -426,13 +427,9 @@ int launch_mt_type(const uint8_t* w, long long row_bytes, const Act& act, YOut y
     hipLaunchKernelGGL((mdec_kernel<TYPE, RT>), dim3(tiles), dim3(256), 0, stream, w, row_bytes, act, y, ldy, M, N);
     return 0;
   }
-  // up to 64 rows: 16-row activation tiles and 64 weight rows per workgroup; prefill: 64
-  // activation rows x 128 weight rows (8 waves)
+  // up to 64 rows: 16-row activation tiles and 64 weight rows per workgroup; prefill: 32 x 32 tiles
   if (M <= 64) return launch_mt<TYPE, 1, 1, 4>(w, row_bytes, act, y, ldy, M, N, stream);
-  constexpr int NT = 1;
-  if constexpr (TYPE == T_Q4_K)
-    if (M > 256) return launch_mt<TYPE, 8, NT, 8>(w, row_bytes, act, y, ldy, M, N, stream);
-  return launch_mt<TYPE, 4, NT, 8>(w, row_bytes, act, y, ldy, M, N, stream);
+  return launch_ptile(TYPE, w, row_bytes, act, y, ldy, M, N, stream);
 }
 
 }  // namespace

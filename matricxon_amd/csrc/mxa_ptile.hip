@@ -1,0 +1,530 @@
+// Prefill matmul (more than 16 activation rows) on the 32 x 32 matrix instructions: Q4_K, Q6_K and
+// Q8_0 weights on Q8_K activations in the workspace.
+//
+// Tiling. A wave owns 32 weight rows x 32 MTW activation rows, a workgroup WN waves along the
+// weight rows: every wave decodes its own weights (once, into registers) and all of them read the
+// workgroup's activation rows from LDS. One v_mfma_i32_32x32x32_i8 covers one 32-value sub-block
+// of Q4_K / Q8_0 (two 16-value sub-blocks of Q6_K): lane l supplies row l % 32 and elements
+// 16 h .. 16 h + 15 of the chunk, h = l / 32, of both operands, and holds weight row n = l % 32 of
+// the results for activation rows m = 8 (i / 4) + 4 h + i % 4, i < 16.
+//
+// Against 16 x 16 tiles each activation byte read from LDS meets twice the weights, and the
+// weights of a chunk are decoded right before the MFMAs that use them, so that only one chunk's
+// operands are live and the decode of one chunk overlaps the MFMAs of another.
+//
+// Copies. A block's 256 bytes of every activation row go straight into LDS (global_load_lds_dwordx4, no
+// registers) in one of two buffers; 16-byte piece c of row r sits at place c ^ (r & 15), so the 32
+// rows of an operand read are spread over all banks without padding. A wave's own weights go into a
+// slot that only it reads: it takes the block into registers and refills the slot at once. Loading
+// the weights per lane into registers instead cost a fifth (Q4_K) to a half (Q6_K) of the time.
+//
+// Bound: instruction issue. Per 32 x 64 x 256 step a Q4_K wave issues 340 VALU instructions (80 a tile
+// to fold, 150 to decode, the rest addresses) and 34 MFMAs of 32 cycles; two waves share a SIMD, the
+// matrix cores are busy 39% of the time, and more stages of copies ahead or another order of the
+// instructions change nothing. Measured on MI355X against the 16 x 16 tiles before (us, kernel alone):
+// Q4_K 14336 x 4096 M = 2048 320 vs 376 (750 TFLOP/s equivalent), Q6_K 4096 x 14336 M = 1024 239 vs 494
+// (its sub-block scales went into two planes: 16 quarter-filled MFMAs and 64 integer products per
+// output quad before), Q8_0 4096 x 4096 M = 2048 111 vs 247, M = 333 36 vs 58.
+//
+// Numerics: integer sums are exact and the fp32 steps are the oracle's, in block order, so the
+// outputs equal the decode kernels' bit for bit.
+#include "mxa_kernels.hpp"
+#include "mxa_tiles.hpp"
+
+#pragma clang fp contract(off)
+
+namespace mxa {
+namespace {
+
+typedef int32_t i32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+__device__ __forceinline__ i32x16 mfma_i8(i32x4 a, i32x4 b, i32x16 c) {
+  return __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, c, 0, 0, 0);
+}
+
+// s_waitcnt lgkmcnt(0): this wave's LDS reads have returned.
+__device__ __forceinline__ void wait_lgkm0() {
+  __builtin_amdgcn_s_waitcnt(0xC07F);
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("" ::: "memory");
+}
+
+constexpr f32x16 kZeroF = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+
+// Integer sums become floats without a conversion. An MFMA chain that starts from kMagic, the bits
+// of 1.5 x 2^23, ends in the bits of the float 1.5 x 2^23 + sum, exactly, while |sum| < 2^22. Two planes
+// hi and lo of weight S (a power of two) then give float(S hi + lo), rounded once as the integer
+// conversion rounds it, by fma(hi', S, -(S + 1) x 1.5 x 2^23) + lo': the first term is S hi -
+// 1.5 x 2^23, a multiple of S below 2^24 S, hence exact. On gfx950 v_fma_f32, v_add_f32 and
+// v_mul_f32 issue in two cycles per wave, v_cvt_f32_i32 and v_lshl_add_u32 in four.
+constexpr int kMagic = 0x4B400000;
+constexpr float kMagicF = 12582912.0f;
+
+// A value that the compiler keeps in vector registers: an AND with a scalar mask takes four cycles
+// and one with a vector mask two, and a float that it knows to come from a half becomes an operand
+// of v_fma_mix_f32 (four cycles, v_fma_f32 two).
+template <class V>
+__device__ __forceinline__ V in_vgpr(V v) {
+  asm("" : "+v"(v));
+  return v;
+}
+
+__device__ __forceinline__ float as_f32(int v) { return __builtin_bit_cast(float, v); }
+
+// One block of the activations in LDS as a wave's tile mt reads it.
+struct PAct {
+  const uint8_t* q;    // swizzled rows of 256 bytes
+  const uint8_t* bs;   // bsums as fp16, 32 bytes per row
+  const float* d;
+  int r, h;            // lane % 32, lane / 32
+  __device__ __forceinline__ i32x4 a(int mt, int t) const {
+    return __builtin_bit_cast(i32x4, *(const u32x4*)(q + (32 * mt + r) * QK + 16 * ((2 * t + h) ^ (r & 15))));
+  }
+  __device__ __forceinline__ f16x8 b(int mt) const { return *(const f16x8*)(bs + (32 * mt + r) * 32 + 16 * h); }
+  // scales of activation rows 8 q4 + 4 h + 0..3 of tile mt
+  __device__ __forceinline__ f32x4 xd(int mt, int q4) const { return *(const f32x4*)(d + 32 * mt + 8 * q4 + 4 * h); }
+};
+
+// The two-plane types' block, chunk by chunk.
+template <class T, int MTW>
+__device__ __forceinline__ void two_planes(const typename T::W& w, const PAct& A, const i32x16& magic, f32x16* acc) {
+  const typename T::S s = T::scales(w);
+  const uint32_t m4 = in_vgpr(0x0F0F0F0Fu);
+  i32x16 hi[MTW], lo[MTW];
+#pragma unroll
+  for (int mt = 0; mt < MTW; ++mt) hi[mt] = lo[mt] = magic;
+#pragma unroll
+  for (int t = 0; t < 8; ++t) {
+    i32x4 bh, bl;
+    T::planes(w, s, t, m4, A.h, bh, bl);
+#pragma unroll
+    for (int mt = 0; mt < MTW; ++mt) {
+      const i32x4 a = A.a(mt, t);
+      hi[mt] = mfma_i8(a, bh, hi[mt]);
+      lo[mt] = mfma_i8(a, bl, lo[mt]);
+    }
+  }
+  const typename T::F f = T::folds(w, s, A.h);
+#pragma unroll
+  for (int mt = 0; mt < MTW; ++mt) T::fold(f, A, mt, hi[mt], lo[mt], acc[mt]);
+}
+
+// Every type: W, a lane's bytes of one block of its weight row; load(lds, off, h), from the wave's
+// slot; and block<MTW>, which folds the block into the outputs of the wave's tiles.
+struct PQ4 {
+  static constexpr bool kBsums = true;
+  struct W {
+    u32x4a4 hdr, q[4];
+  };
+  static constexpr int kBytes = 144;
+  static constexpr bool kShifts = false;
+  __device__ __forceinline__ static W load(const uint8_t* lds, int off, int h) {
+    const uint8_t* p = lds + off;
+    W w;
+    w.hdr = ld16(p);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) w.q[c] = ld16(p + 16 + 32 * c + 16 * h);
+    return w;
+  }
+  struct S {
+    K4Scales s;
+  };
+  __device__ __forceinline__ static S scales(const W& w) { return S{k4_scales(w.hdr.y, w.hdr.z, w.hdr.w)}; }
+  // chunk t's planes: u * sc = 8 (u * (sc >> 3)) + u * (sc & 7), each at most 105
+  __device__ __forceinline__ static void planes(const W& w, const S& s, int t, uint32_t m4, int, i32x4& bh, i32x4& bl) {
+    const uint32_t sc = k4_pick(s.s.sc_lo, s.s.sc_hi, t), sh = sc >> 3, sl = sc & 7;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const uint32_t q = w.q[t >> 1][i], u = ((t & 1) ? q >> 4 : q) & m4;
+      bh[i] = (int)mul_bytes(u, sh);
+      bl[i] = (int)mul_bytes(u, sl);
+    }
+  }
+  struct F {
+    f16x8 bm;
+    float d, dmin, k9;
+  };
+  __device__ __forceinline__ static F folds(const W& w, const S& s, int h) {
+    // summ = sum of min_{j / 2} * bsum_j over the 16 bsums, exact in one fp16 MFMA
+    const uint32_t mn = h ? s.s.mn_hi : s.s.mn_lo;
+    F f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) f.bm[2 * j] = f.bm[2 * j + 1] = (_Float16)(float)((mn >> (8 * j)) & 0xFFu);
+    f.d = in_vgpr(half_to_float(w.hdr.x)), f.dmin = in_vgpr(half_to_float(w.hdr.x >> 16));
+    f.k9 = in_vgpr(-9.0f * kMagicF);
+    return f;
+  }
+  __device__ __forceinline__ static void fold(const F& f, const PAct& A, int mt, const i32x16& hi,
+                                              const i32x16& lo, f32x16& acc) {
+    const f32x16 summ = __builtin_amdgcn_mfma_f32_32x32x16_f16(A.b(mt), f.bm, kZeroF, 0, 0, 0);
+#pragma unroll
+    for (int q4 = 0; q4 < 4; ++q4) {
+      const f32x4 xd = A.xd(mt, q4);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int i = 4 * q4 + e;
+        const float sumi = fmaf(as_f32(hi[i]), 8.0f, f.k9) + as_f32(lo[i]);
+        acc[i] = fmaf(xd[e], fmaf(f.d, sumi, -(f.dmin * summ[i])), acc[i]);
+      }
+    }
+  }
+  template <int MTW>
+  __device__ __forceinline__ static void block(const W& w, const PAct& A, const i32x16& magic, f32x16* acc) {
+    two_planes<PQ4, MTW>(w, A, magic, acc);
+  }
+};
+
+struct PQ6 {
+  static constexpr bool kBsums = false;
+  struct W {
+    u32x4a4 ql[4], qh[2], sc;  // ql[64 hh + 32 q + 16 h ..] at 2 hh + q, qh[32 hh + 16 h ..]
+    uint32_t d;
+  };
+  static constexpr int kBytes = 210;
+  static constexpr bool kShifts = true;
+  // 16 bytes from a 2-byte aligned place, by dwords and v_alignbyte (sh = 0 takes no byte of e)
+  __device__ __forceinline__ static u32x4a4 ld16_a2(const uint8_t* base, uint32_t sh) {
+    const u32x4a4 v = ld16(base);
+    const uint32_t e = ld4(base + 16);
+    return u32x4a4{__builtin_amdgcn_alignbyte(v.y, v.x, sh), __builtin_amdgcn_alignbyte(v.z, v.y, sh),
+                   __builtin_amdgcn_alignbyte(v.w, v.z, sh), __builtin_amdgcn_alignbyte(e, v.w, sh)};
+  }
+  __device__ __forceinline__ static W load(const uint8_t* lds, int off, int h) {
+    const uint32_t sh = (uint32_t)(off & 2);
+    const uint8_t* p = lds + (off & ~3);
+    W w;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) w.ql[c] = ld16_a2(p + 32 * c + 16 * h, sh);
+#pragma unroll
+    for (int c = 0; c < 2; ++c) w.qh[c] = ld16_a2(p + 128 + 32 * c + 16 * h, sh);
+    const u32x4a4 v = ld16(p + 192);
+    const uint32_t e = ld4(p + 208);
+    w.sc = u32x4a4{__builtin_amdgcn_alignbyte(v.y, v.x, sh), __builtin_amdgcn_alignbyte(v.z, v.y, sh),
+                   __builtin_amdgcn_alignbyte(v.w, v.z, sh), __builtin_amdgcn_alignbyte(e, v.w, sh)};
+    w.d = e >> (8 * sh);
+    return w;
+  }
+  struct S {};
+  __device__ __forceinline__ static S scales(const W&) { return S{}; }
+  __device__ __forceinline__ static void planes(const W& w, const S&, int t, uint32_t m4, int h, i32x4& bh, i32x4& bl) {
+    // chunk t = elements 32 t .. of half hh = t / 4, quarter r = t % 4; this lane's sixteen share
+    // scale 2 t + h. p = (u - 32) * sc is 13 bits: p + 128 in 16 bits, its high byte the plane
+    // of 256, its low byte less 128 the plane of 1
+    const int hh = t >> 2, r = t & 3;
+    const uint32_t sw = w.sc[t >> 1] >> (16 * (t & 1));
+    const int sc = (int)(int8_t)(uint8_t)(h ? sw >> 8 : sw);
+    const u16x2 s2 = {(uint16_t)sc, (uint16_t)sc};
+    const uint16_t c0 = (uint16_t)(128 - 32 * sc);
+    const u16x2 c2 = {c0, c0};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const uint32_t l = w.ql[2 * hh + (r & 1)][i], g = w.qh[hh][i];
+      const uint32_t u = r == 0 ? q6_codes<0>(l, g) : r == 1 ? q6_codes<1>(l, g)
+                       : r == 2 ? q6_codes<2>(l, g) : q6_codes<3>(l, g);
+      const u16x2 ue = __builtin_bit_cast(u16x2, u & 0x00FF00FFu);
+      const u16x2 uo = __builtin_bit_cast(u16x2, __builtin_amdgcn_perm(0u, u, 0x0C030C01u));
+      const uint32_t pe = __builtin_bit_cast(uint32_t, (u16x2)(ue * s2 + c2));
+      const uint32_t po = __builtin_bit_cast(uint32_t, (u16x2)(uo * s2 + c2));
+      bh[i] = (int)__builtin_amdgcn_perm(po, pe, 0x07030501u);
+      bl[i] = (int)(__builtin_amdgcn_perm(po, pe, 0x06020400u) ^ 0x80808080u);
+    }
+  }
+  struct F {
+    float d, k257;
+  };
+  __device__ __forceinline__ static F folds(const W& w, const S&, int) {
+    return F{in_vgpr(half_to_float(w.d)), in_vgpr(-257.0f * kMagicF)};
+  }
+  __device__ __forceinline__ static void fold(const F& f, const PAct& A, int mt, const i32x16& hi,
+                                              const i32x16& lo, f32x16& acc) {
+#pragma unroll
+    for (int q4 = 0; q4 < 4; ++q4) {
+      const f32x4 xd = A.xd(mt, q4);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int i = 4 * q4 + e;
+        const float sumi = fmaf(as_f32(hi[i]), 256.0f, f.k257) + as_f32(lo[i]);
+        acc[i] = fmaf(xd[e] * f.d, sumi, acc[i]);
+      }
+    }
+  }
+  template <int MTW>
+  __device__ __forceinline__ static void block(const W& w, const PAct& A, const i32x16& magic, f32x16* acc) {
+    two_planes<PQ6, MTW>(w, A, magic, acc);
+  }
+};
+
+struct PQ8 {
+  static constexpr bool kBsums = false;
+  struct W {
+    // blocks 2 j and 2 j + 1 are 68 bytes from 68 j: d, 32 quants, d, 32 quants; this lane's half
+    // of the even one's quants starts in the upper half of dword 4 h, the odd one's at dword 9 + 4 h
+    u32x4a4 e[4], o[4];
+    uint32_t x[4];  // dword 4 h + 4: the end of the even quants (h = 1: and the odd block's d)
+  };
+  static constexpr int kBytes = 272;
+  static constexpr bool kShifts = false;
+  __device__ __forceinline__ static W load(const uint8_t* lds, int off, int h) {
+    const uint8_t* p = lds + off + 16 * h;
+    W w;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      w.e[j] = ld16(p + 68 * j);
+      w.x[j] = ld4(p + 68 * j + 16);
+      w.o[j] = ld16(p + 68 * j + 36);
+    }
+    return w;
+  }
+  template <int MTW>
+  __device__ __forceinline__ static void block(const W& w, const PAct& A, const i32x16& magic, f32x16* acc) {
+    const float kb = in_vgpr(kMagicF);
+    i32x4 bq[8];
+    float dk[8];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      // lanes of h = 0 hold the even block's d (dword 0), those of h = 1 the odd one's (dword 8)
+      const uint32_t mine = A.h ? w.x[j] >> 16 : w.e[j].x & 0xFFFFu;
+      const uint32_t other = (uint32_t)__shfl_xor((int)mine, 32, 64);
+      dk[2 * j] = in_vgpr(half_to_float(A.h ? other : mine));
+      dk[2 * j + 1] = in_vgpr(half_to_float(A.h ? mine : other));
+      const uint32_t ev[5] = {w.e[j].x, w.e[j].y, w.e[j].z, w.e[j].w, w.x[j]};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        bq[2 * j][i] = (int)__builtin_amdgcn_alignbyte(ev[i + 1], ev[i], 2);
+        bq[2 * j + 1][i] = (int)w.o[j][i];
+      }
+    }
+    // tile by tile, the sums of two blocks open at a time
+#pragma unroll
+    for (int mt = 0; mt < MTW; ++mt) {
+      f32x16 bs = kZeroF;
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        const i32x16 p = mfma_i8(A.a(mt, k), bq[k], magic);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) bs[i] = fmaf(dk[k], as_f32(p[i]) - kb, bs[i]);
+        asm("" : "+v"(bs));
+      }
+#pragma unroll
+      for (int q4 = 0; q4 < 4; ++q4) {
+        const f32x4 xd = A.xd(mt, q4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[mt][4 * q4 + e] = fmaf(xd[e], bs[4 * q4 + e], acc[mt][4 * q4 + e]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+};
+
+template <int TYPE>
+struct PTileOf;
+template <> struct PTileOf<T_Q4_K> { using T = PQ4; };
+template <> struct PTileOf<T_Q6_K> { using T = PQ6; };
+template <> struct PTileOf<T_Q8_0> { using T = PQ8; };
+
+// LDS bytes of one block of `rows` activation rows: q8 | bsums (fp16) | d.
+constexpr int pbuf_bytes(int rows) { return rows * (QK + 32 + 4); }
+// 16-byte pieces that cover one block of a weight row wherever it starts in its first piece, and a
+// wave's LDS bytes for the 32 rows it owns (whole copies of 64 pieces).
+template <class T>
+__host__ __device__ constexpr int ppieces(bool aligned) {
+  return (T::kBytes + (T::kShifts ? 14 : aligned ? 0 : 12) + 15) / 16;
+}
+constexpr int pslot_bytes(int pieces) { return (32 * pieces + 63) / 64 * 1024; }
+
+template <int TYPE, int WN, int MTW>
+__device__ __forceinline__ void ptile_rows(const uint8_t* w, long long row_bytes, const Act& act, YOut y,
+                                           long long ldy, int M, int N, int pieces, int wg, int n_wg, int mg) {
+  using T = typename PTileOf<TYPE>::T;
+  constexpr int kRows = 32 * MTW, kThreads = 64 * WN, kBuf = pbuf_bytes(kRows);
+  extern __shared__ __align__(16) uint8_t smem[];  // two buffers
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r = lane & 31, h = lane >> 5;
+  const int n0 = (xcd_tile(wg, n_wg) * WN + wave) * 32, n = n0 + r;
+  const int m0 = mg * kRows;
+  const int nb = act.nb;
+
+  // The wave's weights: piece c of row q is copied from the 16-byte boundary at or below the
+  // block's start, so every piece holds at least one byte of the block and none lies outside the
+  // 16-byte units that the matrix occupies. Only this wave reads its slot.
+  const uint8_t* wbase = (const uint8_t*)((uintptr_t)w & ~(uintptr_t)15);
+  const uint32_t mis = (uint32_t)((uintptr_t)w & 15);
+  const int slot = 2 * kBuf + wave * pslot_bytes(pieces);
+  const uint32_t slot0 = lds_addr(smem) + slot;
+  const long long row0 = (long long)min(n0, N - 1) * row_bytes;
+  constexpr int kWMax = (32 * ppieces<T>(false) + 63) / 64;
+  const int wcopies = (32 * pieces + 63) / 64;
+  uint32_t woff[kWMax], wpc[kWMax];
+#pragma unroll
+  for (int i = 0; i < kWMax; ++i) {
+    const int s = min(64 * i + lane, 32 * pieces - 1), q = s / pieces;
+    wpc[i] = 16 * (uint32_t)(s - q * pieces);
+    woff[i] = mis + (uint32_t)((min(n0 + q, N - 1) - min(n0, N - 1)) * row_bytes) + (uint32_t)(row0 & 15);
+  }
+  const uint8_t* wrow0 = wbase + (row0 & ~15LL);
+  const int my_piece0 = slot + r * pieces * 16;
+  const uint32_t my_off = mis + (uint32_t)((min(n, N - 1) - min(n0, N - 1)) * row_bytes) + (uint32_t)(row0 & 15);
+  auto copy_w = [&](int b) {
+#pragma unroll
+    for (int i = 0; i < kWMax; ++i)
+      if (i < wcopies)
+        copy16_to_lds_s(wrow0, ((woff[i] + (uint32_t)(T::kBytes * b)) & ~15u) + wpc[i],
+                        (uint32_t)__builtin_amdgcn_readfirstlane((int)(slot0 + 1024 * i)));
+  };
+  auto load_w = [&](int b) {
+    return T::load(smem, my_piece0 + (int)((my_off + (uint32_t)(T::kBytes * b)) & 15u), h);
+  };
+
+  // this wave's copies of a block: 4 rows x 16 pieces each (rows >= M repeat row M - 1)
+  constexpr int kCopies = kRows / 4 / WN;
+  static_assert(kCopies * 4 * WN == kRows, "whole copies per wave");
+  const int8_t* src[kCopies];
+#pragma unroll
+  for (int c = 0; c < kCopies; ++c) {
+    const int rr = 4 * (wave * kCopies + c) + (lane >> 4);
+    src[c] = act.q + (size_t)min(m0 + rr, M - 1) * act.k + 16 * ((lane & 15) ^ (rr & 15));
+  }
+  const uint32_t lds0 = lds_addr(smem);
+  auto copy_q = [&](int b, int buf) {
+#pragma unroll
+    for (int c = 0; c < kCopies; ++c)
+      copy16_to_lds(src[c] + (size_t)b * QK,
+                    (uint32_t)__builtin_amdgcn_readfirstlane(
+                        (int)(lds0 + buf * kBuf + (wave * kCopies + c) * 4 * QK)));
+  };
+  // bsums (16 bytes = half a block per thread) and scales through registers
+  constexpr int kBPer = (2 * kRows + kThreads - 1) / kThreads;
+  constexpr int kDPer = (kRows + kThreads - 1) / kThreads;
+  u32x4a4 sb[kBPer];
+  float sd[kDPer];
+  auto load_s = [&](int b) {
+    if constexpr (T::kBsums) {
+#pragma unroll
+      for (int j = 0; j < kBPer; ++j) {
+        const int p = min(tid + kThreads * j, 2 * kRows - 1);
+        sb[j] = ld16((const uint8_t*)(act.bsums + ((size_t)min(m0 + (p >> 1), M - 1) * nb + b) * 16) + 16 * (p & 1));
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < kDPer; ++j)
+      sd[j] = act.d[(size_t)min(m0 + min(tid + kThreads * j, kRows - 1), M - 1) * nb + b];
+  };
+  auto store_s = [&](int buf) {
+    uint8_t* bs = smem + buf * kBuf + kRows * QK;
+    float* dd = (float*)(bs + kRows * 32);
+    if constexpr (T::kBsums) {
+#pragma unroll
+      for (int j = 0; j < kBPer; ++j) {
+        const int p = tid + kThreads * j;
+        if (p < 2 * kRows) {
+          f16x8 hv;  // exact: |bsum| <= 2032
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            hv[2 * i] = (_Float16)(float)(int16_t)(sb[j][i] & 0xFFFFu);
+            hv[2 * i + 1] = (_Float16)(float)(int16_t)(sb[j][i] >> 16);
+          }
+          *(f16x8*)(bs + 16 * p) = hv;
+        }
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < kDPer; ++j)
+      if (tid + kThreads * j < kRows) dd[tid + kThreads * j] = sd[j];
+  };
+
+  f32x16 acc[MTW];
+#pragma unroll
+  for (int mt = 0; mt < MTW; ++mt) acc[mt] = kZeroF;
+
+  i32x16 magic;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) magic[i] = kMagic;
+  magic = in_vgpr(magic);
+  load_s(0);
+  copy_q(0, 0);
+  copy_w(0);
+  store_s(0);
+  wait_vmcnt(0);
+  __syncthreads();
+  for (int b = 0; b < nb; ++b) {
+    const int buf = b & 1;
+    const bool more = b + 1 < nb;
+    const typename T::W cur = load_w(b);
+    if (more) {
+      load_s(b + 1);
+      copy_q(b + 1, buf ^ 1);
+      wait_lgkm0();  // the weights are in registers: their slot takes the next block's
+      copy_w(b + 1);
+    }
+    const uint8_t* base = smem + buf * kBuf;
+    const PAct A{base, base + kRows * QK, (const float*)(base + kRows * (QK + 32)), r, h};
+    T::template block<MTW>(cur, A, magic, acc);
+    // the folds stay with their MFMAs (left alone, the compiler moves them past the next branch)
+#pragma unroll
+    for (int mt = 0; mt < MTW; ++mt) asm volatile("" : "+v"(acc[mt]));
+    if (more) store_s(buf ^ 1);
+    wait_vmcnt(0);    // this wave's pieces of the next block are in LDS
+    __syncthreads();  // everyone's are, and everyone is done with this block
+  }
+  if (n < N) {
+#pragma unroll
+    for (int mt = 0; mt < MTW; ++mt)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int m = m0 + 32 * mt + 8 * (i >> 2) + 4 * h + (i & 3);
+        if (m < M) y.put((size_t)m * ldy + n, acc[mt][i]);
+      }
+  }
+}
+
+template <int TYPE, int WN, int MTW>
+__global__ __launch_bounds__(64 * WN, 2) void ptile_kernel(const uint8_t* w, long long row_bytes, Act act,
+                                                           YOut y, long long ldy, int M, int N,
+                                                           int pieces) {
+  ptile_rows<TYPE, WN, MTW>(w, row_bytes, act, y, ldy, M, N, pieces, blockIdx.x, gridDim.x, blockIdx.y);
+}
+
+template <int TYPE, int WN, int MTW>
+int launch_p(const uint8_t* w, long long row_bytes, const Act& act, YOut y, long long ldy, int M, int N,
+             hipStream_t stream) {
+  const bool aligned = ((uintptr_t)w & 15) == 0 && row_bytes % 16 == 0;
+  const int pieces = ppieces<typename PTileOf<TYPE>::T>(aligned);
+  const int lds = 2 * pbuf_bytes(32 * MTW) + WN * pslot_bytes(pieces);
+  allow_lds((const void*)ptile_kernel<TYPE, WN, MTW>, lds);
+  const dim3 grid((N + 32 * WN - 1) / (32 * WN), (M + 32 * MTW - 1) / (32 * MTW));
+  hipLaunchKernelGGL((ptile_kernel<TYPE, WN, MTW>), grid, dim3(64 * WN), lds, stream, w, row_bytes, act, y,
+                     ldy, M, N, pieces);
+  return 0;
+}
+
+// Waves along the weight rows and activation tiles per wave. Two tiles share a wave's decoded weights,
+// eight waves an activation block in LDS, as long as the grid still fills the chip: measured on
+// MI355X (us, kernel alone, 8 x 2 / 4 x 2 / 2 x 1 waves x tiles): Q4_K 14336 x 4096 M = 2048
+// 326 / 336 / 446, 4096 x 4096 M = 1024 46.0 / 47.7 / 69, M = 128 41 / 28 / 20; Q6_K 4096 x 14336
+// M = 1024 239 / 247 / 443; Q8_0 4096 x 4096 M = 2048 114 / 111 / 157, M = 333 56 / 45 / 36.
+template <int TYPE>
+int launch_p_type(const uint8_t* w, long long row_bytes, const Act& act, YOut y, long long ldy, int M, int N,
+                  hipStream_t stream) {
+  const long long m_tiles = (M + 63) / 64, cus = cu_count();
+  if (TYPE != T_Q8_0 && (N + 255) / 256 * m_tiles >= cus)
+    return launch_p<TYPE, 8, 2>(w, row_bytes, act, y, ldy, M, N, stream);
+  if ((N + 127) / 128 * m_tiles >= (TYPE == T_Q8_0 ? cus * 3 / 2 : cus * 3 / 4))
+    return launch_p<TYPE, 4, 2>(w, row_bytes, act, y, ldy, M, N, stream);
+  return launch_p<TYPE, 2, 1>(w, row_bytes, act, y, ldy, M, N, stream);
+}
+
+}  // namespace
+
+int launch_ptile(int type, const uint8_t* w, long long row_bytes, const Act& act, YOut y, long long ldy,
+                 int m_rows, int n_rows, hipStream_t stream) {
+  switch (type) {
+    case T_Q4_K: return launch_p_type<T_Q4_K>(w, row_bytes, act, y, ldy, m_rows, n_rows, stream);
+    case T_Q6_K: return launch_p_type<T_Q6_K>(w, row_bytes, act, y, ldy, m_rows, n_rows, stream);
+    case T_Q8_0: return launch_p_type<T_Q8_0>(w, row_bytes, act, y, ldy, m_rows, n_rows, stream);
+    default: return -1;
+  }
+}
+
+}  // namespace mxa

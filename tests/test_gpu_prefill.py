@@ -1,0 +1,69 @@
+"""The prefill tiles (mxa_ptile.hip) at the places where they can go wrong, against the oracle bit for
+bit: remainders of the 32-row tiles on both sides, one block per row, rows whose blocks start at
+2-byte boundaries, weights that start 4 bytes past a 16-byte boundary, each choice of workgroup, and
+the largest integer sums of each type."""
+
+import numpy as np
+import pytest
+import torch
+
+from matricxon_amd import synthetic as S
+from oracle import dequant as D
+from tests.test_gpu_kernels import bits, dev, host
+
+pytestmark = pytest.mark.gpu
+
+TYPES = [D.Q4_K, D.Q6_K, D.Q8_0]
+
+
+def check(gpu, oracle, t, w, x, n, k, shift=0):
+    buf = torch.zeros(w.size + 64, dtype=torch.uint8, device="cuda")
+    wd = buf[shift:shift + w.size].view(n, -1)
+    wd.copy_(dev(w))
+    assert wd.data_ptr() % 16 == shift
+    got = host(gpu.matmul(t, wd, dev(x), n, k))
+    rows = np.unique(np.concatenate([np.arange(min(n, 200)), np.arange(max(0, n - 200), n), np.arange(0, n, 37)]))
+    want = oracle.gemm(t, w[rows], x, len(rows), k)
+    assert np.array_equal(bits(got[:, rows]), bits(want))
+
+
+@pytest.mark.parametrize("t", TYPES)
+@pytest.mark.parametrize("n,k,m", [
+    (1, 256, 65), (31, 256, 96), (33, 512, 97), (64, 768, 128), (129, 1280, 129), (257, 2816, 200),
+    (1000, 1024, 333),   # two waves, one tile
+    (8200, 256, 210),    # four waves, two tiles
+    (16500, 512, 300),   # eight waves, two tiles
+])
+def test_prefill_tiles_match_oracle(gpu, oracle, t, n, k, m) -> None:
+    w = S.packed_weight(t, n, k, seed=n + k)
+    check(gpu, oracle, t, w, S.activations(m, k, seed=m), n, k)
+
+
+@pytest.mark.parametrize("t", TYPES)
+@pytest.mark.parametrize("shift", [4, 8, 12])
+def test_prefill_weight_alignment(gpu, oracle, t, shift) -> None:
+    w = S.packed_weight(t, 70, 1280, seed=9)
+    check(gpu, oracle, t, w, S.activations(70, 1280, seed=10), 70, 1280, shift)
+
+
+@pytest.mark.parametrize("t", TYPES)
+@pytest.mark.parametrize("sign", [1, -1])
+def test_prefill_largest_sums(gpu, oracle, t, sign) -> None:
+    """Every code, scale and activation at its largest magnitude, all products of one sign: the sums
+    that the float conversion of the integer planes has to hold."""
+    n, k, m = 40, 512, 80
+    w = S.packed_weight(t, n, k, seed=1).reshape(n, -1)
+    if t == D.Q4_K:
+        b = w.reshape(-1, 144)
+        b[:, 4:16] = 0xFF  # every scale and min 63
+        b[:, 16:] = 0xFF  # every code 15
+    elif t == D.Q6_K:
+        b = w.reshape(-1, 210)
+        b[:, :192] = 0  # every code 0, the value -32
+        b[:, 192:208] = 0x80  # every scale -128
+    else:
+        w.reshape(-1, 34)[:, 2:] = 0x80  # every quant -128
+    x = np.full((m, k), 127.0 * sign, dtype=np.float32)
+    x[1::2] *= -1
+    x[2::5, 3::7] *= -0.5
+    check(gpu, oracle, t, w, x, n, k)
