@@ -201,6 +201,12 @@ int launch_mtile(int type, const uint8_t* w, long long row_bytes, const Act& act
 int launch_ptile(int type, const uint8_t* w, long long row_bytes, const Act& act, YOut y, long long ldy,
                  int m_rows, int n_rows, hipStream_t stream);
 
+// Grouped MoE projection on the prefill tiles, chunks of 32 or 64 rows of each expert; -1 when the work
+// list is too long.
+int launch_moe_ptile(int type, const uint8_t* w, long long row_bytes, long long expert_stride, int n_experts,
+                     const Act& act, const int32_t* offsets, int total_rows, YOut y, long long ldy, int n_rows,
+                     hipStream_t stream);
+
 // Grouped MoE projection (mxa_mtile.hip): expert e of n_experts multiplies rows
 // [offsets[e], offsets[e + 1]) of the total_rows Q8_K activation rows in `act` (a device array of
 // n_experts + 1 ascending offsets; at most max_rows rows per expert) by its packed weight

@@ -207,33 +207,6 @@ __global__ __launch_bounds__(64 * WAVES) void mtile_kernel(const uint8_t* w, lon
                                   blockIdx.y);
 }
 
-// Grouped MoE projection on the row-tiled body: every expert's rows [offsets[e], offsets[e + 1])
-// (clamped into [0, total_rows), as moe_dec_kernel below clamps them) are cut into chunks of 16 MT
-// rows, and workgroup z of the grid's third dimension takes item z of the list of (expert, chunk)
-// pairs, experts in order, so a weight tile is read once per 16 MT rows of its expert instead of
-// once per 16. Every wave finds its item from the offset table (lane l counts the chunks of
-// experts 4 l .. 4 l + 3, a wave prefix sum locates item z), so the list covers every row whatever
-// the routing: an expert that a token names twice has more rows than tokens, and the host sizes
-// the grid by n_experts + ceil(total_rows / (16 MT)), which bounds the list's length. A workgroup
-// past the list's end exits. n_experts <= 256. (One chunk per workgroup: a loop over chunks made
-// the Q6_K body spill.)
-template <int TYPE, int MT, int NT, int WAVES>
-__global__ __launch_bounds__(64 * WAVES) void moe_mtile_kernel(const uint8_t* w, long long row_bytes,
-                                                               long long expert_stride, Act act,
-                                                               const int32_t* __restrict__ offsets,
-                                                               int n_experts, int total_rows, YOut y,
-                                                               long long ldy, int N) {
-  int e, p0, M;
-  // past the list: uniform over the workgroup, before any barrier
-  if (!moe_chunk_item(offsets, n_experts, total_rows, 16 * MT, blockIdx.z, e, p0, M)) return;
-  Act a = act;
-  a.q = act.q + (size_t)p0 * act.k;
-  a.d = act.d + (size_t)p0 * act.nb;
-  a.bsums = act.bsums + (size_t)p0 * act.nb * 16;
-  mtile_rows<TYPE, MT, NT, WAVES>(w + (size_t)e * expert_stride, row_bytes, a,
-                                  y.at((size_t)p0 * ldy), ldy, M, N, blockIdx.x, gridDim.x, 0);
-}
-
 // Batched decode (M <= 16): 32 weight rows per workgroup and the blocks of each chunk split over
 // the 4 waves (wave w takes blocks w and w + 4 of an 8-block chunk, for both 16-row tiles), so that
 // N = 4096..14336 still gives the GPU 128..448 workgroups. The block values go through LDS and are
@@ -444,55 +417,32 @@ int launch_moe_dec(int type, const uint8_t* w, long long row_bytes, long long ex
     return -1;
   const int chunks = (max_rows + 15) / 16;
   if (chunks > 65535) return -1;
-  // Past 32 rows per expert (the bound), 64-row chunks through the prefill tile body read each
-  // weight tile once per 64 rows instead of once per 16 (measured on MI355X, eager forward at
-  // 128 tokens, the same bits: 8 experts top 2, 4096 x 14336, 607 vs 1058 us; 40 experts top 8,
-  // 1536 x 512, 99-113 vs 176 us; at 16 tokens both forms tie)
-  // Up to 32 rows, expert matrices of 4096 rows and more take 16-row chunks through the same body
-  // (64 weight rows per 4-wave workgroup): same box, forward only, 8 experts top 2 (4096 x 14336),
-  // 8 / 16 / 24 / 32 tokens 404 / 392 / 406 / 410 vs 443 / 429 / 441 / 445 us on the decode tile;
-  // the 40 small experts (512 and 1536 rows) tie or lose, so they keep the decode tile.
-  constexpr int kMoeMtileMinRows = 32, kMoeSmallTileMinN = 4096;
-  // mt activation tiles and `waves` waves of 16 weight rows per workgroup; the grid's third
-  // dimension bounds the (expert, chunk) list whatever the per-expert counts
-  auto go_mt = [&](auto k_q4, auto k_q8, auto k_q6, int mt, int waves, int lds) {
-    const int rows = 16 * mt, wg_rows = 16 * waves;
-    const dim3 grid((n_rows + wg_rows - 1) / wg_rows, 1, n_experts + (total_rows + rows - 1) / rows);
-    auto run = [&](auto kern) {
-      allow_lds((const void*)kern, lds);
-      hipLaunchKernelGGL(kern, grid, dim3(64 * waves), lds, stream, w, row_bytes, expert_stride,
-                         act, offsets, n_experts, total_rows, y, ldy, n_rows);
-      return 0;
-    };
-    switch (type) {
-      case T_Q4_K: return run(k_q4);
-      case T_Q8_0: return run(k_q8);
-      case T_Q6_K: return run(k_q6);
-      default: return -1;
-    }
-  };
-  // Up to 96 rows per expert, expert matrices of 1024 rows and more take the batched-decode
-  // bodies (short and long rows) in 16-row chunks, the CUs shared among the experts that can have
-  // rows. Measured on MI355X, eager forward of 64 experts top 8 (2048 x 1024) at 4 / 16 / 32 / 64
-  // tokens 100 / 171 / 188 / 204 us against 123 / 170 / 186 / 222 on the decode tile and prefill
-  // tile bodies, 16 experts top 4 (3072 x 2048) 104 / 97 / 109 / 166 against 135 / 131 / 140 /
-  // 178; 8 experts top 2 (4096 x 14336), the same bits:
-  // 16 / 24 / 32 / 48 / 64 / 80 / 96 tokens 304 / 299 / 298 / 538 / 536 / 558 / 545 us against
-  // 395 / 415 / 414 / 571 / 596 / 608 / 598 on the prefill tile bodies; at 112 / 128 tokens the
-  // decode bodies lose (786 / 794 vs 594 / 607 us: more 16-row chunks per expert), so larger bounds
-  // keep the prefill tile body.
+  // The prefill tiles (32- or 64-row chunks, 128 weight rows a workgroup), except
+  // - where the routing gives too few of them to fill the chip, and where the experts of a large matrix
+  //   have two to eight rows on average: the batched-decode bodies (16-row chunks, every CU a share of
+  //   the rows, all of it requested early), if they take the shape;
+  // - few tiles of shapes that those do not take: the decode tile below.
+  // Measured on MI355X, weights from HBM, us, kernel alone, prefill tiles / the other form: 64 experts
+  // top 8, Q4_K 1024 x 2048, 1 token (64 tiles) 13.1 / 8.8, 4 (256) 15.5 / 14.9, 16 (1 row a expert and
+  // more) 22 / 31, Q6_K 2048 x 1024 (decode tile), 2 / 4 / 16 tokens 15 / 27, 22 / 47, 37 / 81; 8 experts
+  // top 2, Q4_K 14336 x 4096, 4 / 16 / 32 / 48 / 96 tokens 52 / 62, 70 / 63, 69 / 63, 73 / 118, 72 / 120,
+  // Q6_K 4096 x 14336, 2 tokens (128 tiles) 134 / 73, 16 138 / 139, 96 138 / 277; 16 experts top 4, Q6_K
+  // 3072 x 2048, 4 / 16 tokens 24 / 33, 38 / 34; 4 experts top 1, Q6_K 14336 x 4096, 8 tokens 67 / 46; 40
+  // experts top 8 (decode tile), Q4_K 512 x 1536, 4 / 16 tokens (128 / 160 tiles) 10.7 / 7.7, 11.0 / 14.7,
+  // Q6_K 1536 x 512, 1 token (96) 8.6 / 15.2.
   constexpr int kMoeDecodeBodyMaxRows = 96, kMoeDecodeBodyMinN = 1024;
-  if (max_rows <= kMoeDecodeBodyMaxRows && n_rows >= kMoeDecodeBodyMinN &&
+  const long long busy = total_rows < n_experts ? total_rows : n_experts;
+  const long long chunks32 = (total_rows + 31) / 32;
+  const long long tiles = (n_rows + 127) / 128 * (busy > chunks32 ? busy : chunks32);
+  const bool streams = n_rows >= 2048 && total_rows >= 2LL * n_experts && total_rows <= 8LL * n_experts;
+  if ((tiles < cu_count() || streams) && max_rows <= kMoeDecodeBodyMaxRows && n_rows >= kMoeDecodeBodyMinN &&
       launch_moe_bwave(type, w, row_bytes, expert_stride, n_experts, act, offsets, total_rows, y,
                        ldy, n_rows, stream) == 0)
     return 0;
-  const bool list_fits = n_experts <= 256 && n_experts + (total_rows + 15) / 16 <= 65535;
-  if (list_fits && max_rows > kMoeMtileMinRows)
-    return go_mt(moe_mtile_kernel<T_Q4_K, 4, 1, 8>, moe_mtile_kernel<T_Q8_0, 4, 1, 8>,
-                 moe_mtile_kernel<T_Q6_K, 4, 1, 8>, 4, 8, 2 * kMtBuf<4>);
-  if (list_fits && n_rows >= kMoeSmallTileMinN)
-    return go_mt(moe_mtile_kernel<T_Q4_K, 1, 1, 4>, moe_mtile_kernel<T_Q8_0, 1, 1, 4>,
-                 moe_mtile_kernel<T_Q6_K, 1, 1, 4>, 1, 4, 2 * kMtBuf<1>);
+  if ((max_rows > 32 || tiles >= (type == T_Q6_K ? 64 : 160)) &&
+      launch_moe_ptile(type, w, row_bytes, expert_stride, n_experts, act, offsets, total_rows, y, ldy, n_rows,
+                       stream) == 0)
+    return 0;
   // Tile groups per workgroup (each group's chunk of activations staged once for all of them):
   // the most of 4, 2, 1 that still gives two workgroups per CU (Q8_0 at most 2: four spill).
   // Measured on MI355X, eager forward of 8 experts top 2 (4096 x 14336; Q4_K gate / up, Q6_K

@@ -333,9 +333,10 @@ __host__ __device__ constexpr int ppieces(bool aligned) {
 }
 constexpr int pslot_bytes(int pieces) { return (32 * pieces + 63) / 64 * 1024; }
 
+// The outputs of activation rows m0 .. m0 + 32 MTW - 1 of M.
 template <int TYPE, int WN, int MTW>
 __device__ __forceinline__ void ptile_rows(const uint8_t* w, long long row_bytes, const Act& act, YOut y,
-                                           long long ldy, int M, int N, int pieces, int wg, int n_wg, int mg) {
+                                           long long ldy, int M, int N, int pieces, int wg, int n_wg, int m0) {
   using T = typename PTileOf<TYPE>::T;
   constexpr int kRows = 32 * MTW, kThreads = 64 * WN, kBuf = pbuf_bytes(kRows);
   extern __shared__ __align__(16) uint8_t smem[];  // two buffers
@@ -343,7 +344,6 @@ __device__ __forceinline__ void ptile_rows(const uint8_t* w, long long row_bytes
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 31, h = lane >> 5;
   const int n0 = (xcd_tile(wg, n_wg) * WN + wave) * 32, n = n0 + r;
-  const int m0 = mg * kRows;
   const int nb = act.nb;
 
   // The wave's weights: piece c of row q is copied from the 16-byte boundary at or below the
@@ -479,11 +479,42 @@ __device__ __forceinline__ void ptile_rows(const uint8_t* w, long long row_bytes
   }
 }
 
+// Two tiles per wave, or one where the second would have no row (the choice stands outside the block
+// loop: inside it, the accumulators' moves cost a tenth of the time).
+template <int TYPE, int WN, int MTW>
+__device__ __forceinline__ void ptile_any(const uint8_t* w, long long row_bytes, const Act& act, YOut y,
+                                          long long ldy, int M, int N, int pieces, int wg, int n_wg, int m0) {
+  if (MTW == 2 && m0 + 32 >= M)
+    ptile_rows<TYPE, WN, 1>(w, row_bytes, act, y, ldy, M, N, pieces, wg, n_wg, m0);
+  else
+    ptile_rows<TYPE, WN, MTW>(w, row_bytes, act, y, ldy, M, N, pieces, wg, n_wg, m0);
+}
+
 template <int TYPE, int WN, int MTW>
 __global__ __launch_bounds__(64 * WN, 2) void ptile_kernel(const uint8_t* w, long long row_bytes, Act act,
                                                            YOut y, long long ldy, int M, int N,
                                                            int pieces) {
-  ptile_rows<TYPE, WN, MTW>(w, row_bytes, act, y, ldy, M, N, pieces, blockIdx.x, gridDim.x, blockIdx.y);
+  ptile_any<TYPE, WN, MTW>(w, row_bytes, act, y, ldy, M, N, pieces, blockIdx.x, gridDim.x,
+                           32 * MTW * blockIdx.y);
+}
+
+// Grouped MoE projection: item blockIdx.z of the (expert, chunk of 32 MTW rows) list
+// (moe_chunk_item), workgroups along the expert's weight rows in blockIdx.x.
+template <int TYPE, int WN, int MTW>
+__global__ __launch_bounds__(64 * WN, 2) void moe_ptile_kernel(const uint8_t* w, long long row_bytes,
+                                                               long long expert_stride, Act act,
+                                                               const int32_t* __restrict__ offsets,
+                                                               int n_experts, int total_rows, YOut y,
+                                                               long long ldy, int N, int pieces) {
+  int e, p0, M;
+  // past the list: uniform over the workgroup, before any barrier
+  if (!moe_chunk_item(offsets, n_experts, total_rows, 32 * MTW, blockIdx.z, e, p0, M)) return;
+  Act a = act;
+  a.q = act.q + (size_t)p0 * act.k;
+  a.d = act.d + (size_t)p0 * act.nb;
+  a.bsums = act.bsums + (size_t)p0 * act.nb * 16;
+  ptile_any<TYPE, WN, MTW>(w + (size_t)e * expert_stride, row_bytes, a, y.at((size_t)p0 * ldy), ldy, M, N,
+                           pieces, blockIdx.x, gridDim.x, 0);
 }
 
 template <int TYPE, int WN, int MTW>
@@ -515,7 +546,47 @@ int launch_p_type(const uint8_t* w, long long row_bytes, const Act& act, YOut y,
   return launch_p<TYPE, 2, 1>(w, row_bytes, act, y, ldy, M, N, stream);
 }
 
+template <int TYPE, int WN, int MTW>
+int launch_moe_p(const uint8_t* w, long long row_bytes, long long expert_stride, int n_experts, const Act& act,
+                 const int32_t* offsets, int total_rows, YOut y, long long ldy, int N, hipStream_t stream) {
+  const bool aligned = ((uintptr_t)w & 15) == 0 && row_bytes % 16 == 0 && expert_stride % 16 == 0;
+  const int pieces = ppieces<typename PTileOf<TYPE>::T>(aligned);
+  const int lds = 2 * pbuf_bytes(32 * MTW) + WN * pslot_bytes(pieces);
+  const long long items = n_experts + (total_rows + 32 * MTW - 1) / (32 * MTW);
+  if (n_experts > 256 || items > 65535) return -1;
+  allow_lds((const void*)moe_ptile_kernel<TYPE, WN, MTW>, lds);
+  hipLaunchKernelGGL((moe_ptile_kernel<TYPE, WN, MTW>), dim3((N + 32 * WN - 1) / (32 * WN), 1, (unsigned)items),
+                     dim3(64 * WN), lds, stream, w, row_bytes, expert_stride, act, offsets, n_experts, total_rows,
+                     y, ldy, N, pieces);
+  return 0;
+}
+
+template <int TYPE>
+int launch_moe_p_type(const uint8_t* w, long long row_bytes, long long expert_stride, int n_experts, const Act& act,
+                      const int32_t* offsets, int total_rows, YOut y, long long ldy, int N, hipStream_t stream) {
+  // 64-row chunks once an expert has more than 32 rows on average (MI355X, us, 64- / 32-row chunks:
+  // 64 experts top 8, 512 tokens, Q6_K 2048 x 1024 63 / 78, Q4_K 1024 x 2048 49 / 45; 8 experts top 2
+  // at 256 tokens, Q4_K 14336 x 4096 129 / 150, at 96 tokens 69 / 65)
+  if (total_rows > 32LL * n_experts)
+    return launch_moe_p<TYPE, 4, 2>(w, row_bytes, expert_stride, n_experts, act, offsets, total_rows, y, ldy, N, stream);
+  return launch_moe_p<TYPE, 4, 1>(w, row_bytes, expert_stride, n_experts, act, offsets, total_rows, y, ldy, N, stream);
+}
+
 }  // namespace
+
+int launch_moe_ptile(int type, const uint8_t* w, long long row_bytes, long long expert_stride, int n_experts,
+                     const Act& act, const int32_t* offsets, int total_rows, YOut y, long long ldy, int n_rows,
+                     hipStream_t stream) {
+  auto go = [&](auto f) {
+    return f(w, row_bytes, expert_stride, n_experts, act, offsets, total_rows, y, ldy, n_rows, stream);
+  };
+  switch (type) {
+    case T_Q4_K: return go(launch_moe_p_type<T_Q4_K>);
+    case T_Q6_K: return go(launch_moe_p_type<T_Q6_K>);
+    case T_Q8_0: return go(launch_moe_p_type<T_Q8_0>);
+    default: return -1;
+  }
+}
 
 int launch_ptile(int type, const uint8_t* w, long long row_bytes, const Act& act, YOut y, long long ldy,
                  int m_rows, int n_rows, hipStream_t stream) {

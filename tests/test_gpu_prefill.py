@@ -67,3 +67,20 @@ def test_prefill_largest_sums(gpu, oracle, t, sign) -> None:
     x[1::2] *= -1
     x[2::5, 3::7] *= -0.5
     check(gpu, oracle, t, w, x, n, k)
+
+
+@pytest.mark.parametrize("t", TYPES)
+@pytest.mark.parametrize("counts", [
+    [0, 1, 31, 32, 33, 2],  # 32-row chunks
+    [0, 1, 64, 65, 33, 0, 129],  # 64-row chunks, the last one of some experts with one tile's rows
+])
+def test_grouped_prefill_tiles_match_oracle(gpu, oracle, t, counts) -> None:
+    n, k, e = 300, 1280, len(counts)
+    w = np.stack([S.packed_weight(t, n, k, seed=70 + i) for i in range(e)])
+    x = S.activations(sum(counts), k, seed=71)
+    off = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    got = host(gpu.matmul_moe(t, dev(w), dev(x), dev(off), max(counts), n, k))
+    for i, c in enumerate(counts):
+        if c:
+            rows = slice(off[i], off[i + 1])
+            assert np.array_equal(bits(got[rows]), bits(oracle.gemm(t, w[i], x[rows], n, k)))
