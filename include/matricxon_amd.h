@@ -319,6 +319,14 @@ int mxa_dequantize(int ggml_type, const void *blocks, long long n_blocks, float 
 int mxa_dequant_rows(int ggml_type, const void *w, long long n_src_rows, const int32_t *rows,
                      int n_rows, int row_width, float *out, void *stream);
 
+/* The rows of a packed embedding for n_ids token ids (a DEVICE int64 array, 8-byte aligned; a negative
+ * id counts from the end, as torch indexes; an id outside [-n_src_rows, n_src_rows) gives a row of
+ * NaN), in one launch: out (n_ids, row_width), 16-byte aligned, float32, or with out_bf16 != 0
+ * bfloat16, each value the bit-exact float32 one rounded as torch's cast rounds it.
+ * Replaces the lookup of `DevicePackedEmbedding.forward` (app/architectures/device_packed.py:81-84). */
+int mxa_embed_rows(int ggml_type, const void *w, long long n_src_rows, const int64_t *ids, int n_ids,
+                   int row_width, void *out, int out_bf16, void *stream);
+
 /* Reorders packed rows on the device: dst row i = src row order[i] for i < n_rows, rows of
  * row_bytes bytes (any GGUF type: a row is whole blocks); `order` is a device int32 array; an
  * index outside [0, n_src_rows) gives a row of zero bytes. src and dst must not overlap.

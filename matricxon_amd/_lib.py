@@ -38,6 +38,7 @@ EXPORTS = (
     "mxa_silu_mul_q8_k",
     "mxa_dequantize",
     "mxa_dequant_rows",
+    "mxa_embed_rows",
     "mxa_gather_rows",
     "mxa_stream_read",
     "mxa_last_error",
@@ -136,6 +137,8 @@ def load() -> ctypes.CDLL:
     lib.mxa_dequantize.restype = _i
     lib.mxa_dequant_rows.argtypes = [_i, _vp, _ll, _vp, _i, _i, _vp, _vp]
     lib.mxa_dequant_rows.restype = _i
+    lib.mxa_embed_rows.argtypes = [_i, _vp, _ll, _vp, _i, _i, _vp, _i, _vp]
+    lib.mxa_embed_rows.restype = _i
     lib.mxa_gather_rows.argtypes = [_vp, _ll, _ll, _vp, _i, _vp, _vp]
     lib.mxa_gather_rows.restype = _i
     lib.mxa_stream_read.argtypes = [_vp, _ll, _vp, _vp]

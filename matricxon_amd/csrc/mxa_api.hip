@@ -577,8 +577,8 @@ int mxa_dequantize(int ggml_type, const void* blocks, long long n_blocks, float*
                    void* stream) {
   if (!known_type(ggml_type) || blocks == nullptr || out == nullptr || n_blocks <= 0)
     return MXA_ERR_UNSUPPORTED;
-  if (mxa::launch_dequant(ggml_type, (const uint8_t*)blocks, nullptr, 0, 0, 1, n_blocks, out,
-                          (hipStream_t)stream) != 0)
+  if (mxa::launch_dequant(ggml_type, (const uint8_t*)blocks, nullptr, nullptr, 0, 0, 1, n_blocks,
+                          mxa::YOut::f32(out), (hipStream_t)stream) != 0)
     return MXA_ERR_UNSUPPORTED;
   return check_launch();
 }
@@ -590,8 +590,22 @@ int mxa_dequant_rows(int ggml_type, const void* w, long long n_src_rows, const i
     return MXA_ERR_UNSUPPORTED;
   const int bpr = row_width / block_elems(ggml_type);
   const long long rb = (long long)mxa_row_bytes(ggml_type, row_width);
-  if (mxa::launch_dequant(ggml_type, (const uint8_t*)w, rows, n_src_rows, rb, bpr,
-                          (long long)n_rows * bpr, out, (hipStream_t)stream) != 0)
+  if (mxa::launch_dequant(ggml_type, (const uint8_t*)w, rows, nullptr, n_src_rows, rb, bpr,
+                          (long long)n_rows * bpr, mxa::YOut::f32(out), (hipStream_t)stream) != 0)
+    return MXA_ERR_UNSUPPORTED;
+  return check_launch();
+}
+
+int mxa_embed_rows(int ggml_type, const void* w, long long n_src_rows, const int64_t* ids, int n_ids,
+                   int row_width, void* out, int out_bf16, void* stream) {
+  if (!mxa_supports(ggml_type, row_width) || w == nullptr || ids == nullptr || out == nullptr ||
+      n_ids <= 0 || n_src_rows <= 0 || !aligned(ids, 8) || !aligned(out, 16))
+    return MXA_ERR_UNSUPPORTED;
+  const int bpr = row_width / block_elems(ggml_type);
+  const long long rb = (long long)mxa_row_bytes(ggml_type, row_width);
+  if (mxa::launch_dequant(ggml_type, (const uint8_t*)w, nullptr, ids, n_src_rows, rb, bpr,
+                          (long long)n_ids * bpr, out_bf16 ? mxa::YOut::bf16(out) : mxa::YOut::f32((float*)out),
+                          (hipStream_t)stream) != 0)
     return MXA_ERR_UNSUPPORTED;
   return check_launch();
 }

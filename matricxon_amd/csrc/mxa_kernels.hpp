@@ -104,9 +104,11 @@ void launch_gather_rows(const void* src, long long n_src_rows, long long row_byt
                         const int32_t* order, int n_rows, void* dst, hipStream_t stream);
 
 
-int launch_dequant(int type, const uint8_t* base, const int32_t* rows, long long n_src_rows,
-                   long long row_bytes, int blocks_per_row, long long n_blocks, float* out,
-                   hipStream_t stream);
+// Blocks of a flat array (rows and ids null), of the rows `rows`, or of the rows `ids` (a negative id
+// counts from the end); out 16-byte aligned.
+int launch_dequant(int type, const uint8_t* base, const int32_t* rows, const int64_t* ids,
+                   long long n_src_rows, long long row_bytes, int blocks_per_row, long long n_blocks,
+                   YOut out, hipStream_t stream);
 
 // Text that mxa_last_error() returns on the calling thread until the next error.
 void set_last_error(const char* text);

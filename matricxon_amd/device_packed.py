@@ -206,7 +206,7 @@ class DevicePackedLinear(nn.Module):
 
 class DevicePackedEmbedding(nn.Module):
     """Token embeddings kept as packed GGUF rows in device memory. `forward` expands just the
-    looked-up ids (one `mxa_dequant_rows` launch); `as_linear` reuses the same bytes as the tied
+    looked-up ids (one `mxa_embed_rows` launch); `as_linear` reuses the same bytes as the tied
     output projection."""
 
     def __init__(
@@ -226,12 +226,12 @@ class DevicePackedEmbedding(nn.Module):
 
     def forward(self, ids: torch.Tensor) -> torch.Tensor:
         # torch indexing semantics of the reference's `self.packed[ids]` (device_packed.py:81-84):
-        # negative ids count from the end. The wrap runs on the device (no host sync); an id
-        # outside [-num_embeddings, num_embeddings) gives a row of NaN instead of an error.
-        flat = ids.reshape(-1).to(torch.int64)
-        flat = torch.where(flat < 0, flat + self.num_embeddings, flat)
-        rows = self._gemm.dequant_rows(self._ggml_type, self.packed, flat, self.embedding_dim)
-        return rows.reshape(*ids.shape, self.embedding_dim).to(self.dtype)
+        # negative ids count from the end. One launch writes the layer's dtype, with no host sync;
+        # an id outside [-num_embeddings, num_embeddings) gives a row of NaN instead of an error.
+        rows = self._gemm.embed_rows(self._ggml_type, self.packed, ids, self.embedding_dim, self.dtype)
+        if rows.dtype != self.dtype:
+            rows = rows.to(self.dtype)
+        return rows.reshape(*ids.shape, self.embedding_dim)
 
     def as_linear(self) -> DevicePackedLinear:
         return DevicePackedLinear(self.packed, self.embedding_dim, self._ggml_type,

@@ -717,6 +717,27 @@ class HipGemm:
                                            _stream(data.device))
         self._check(status, "mxa_stream_read", 0)
 
+    def embed_rows(self, ggml_type: int, packed: torch.Tensor, ids: torch.Tensor, row_width: int,
+                   dtype: torch.dtype) -> torch.Tensor:
+        """Rows `ids` (integers, any shape) of the packed embedding as (ids.numel(), row_width) in
+        float32, or in bfloat16 for that dtype, in one launch with no host sync. A negative id
+        counts from the end; one outside [-n_rows, n_rows) gives a row of NaN."""
+        ggml_type = int(ggml_type)
+        if not self.supports_dequant_rows(ggml_type, row_width):
+            raise RuntimeError(f"mxa_embed_rows failed with status -1 for type {ggml_type}")
+        self._check_packed(ggml_type, packed, packed.shape[0], row_width)
+        idx = ids.detach().reshape(-1).to(device=packed.device, dtype=torch.int64).contiguous()
+        bf16 = dtype == torch.bfloat16
+        out = torch.empty((idx.shape[0], row_width), dtype=torch.bfloat16 if bf16 else torch.float32,
+                          device=packed.device)
+        if idx.shape[0] == 0:
+            return out
+        status = self._lib.mxa_embed_rows(ggml_type, packed.data_ptr(), packed.shape[0], idx.data_ptr(),
+                                          idx.shape[0], row_width, out.data_ptr(), int(bf16),
+                                          _stream(packed.device))
+        self._check(status, "mxa_embed_rows", ggml_type)
+        return out
+
     def dequant_rows(self, ggml_type: int, packed: torch.Tensor, row_indices: torch.Tensor,
                      row_width: int) -> torch.Tensor:
         """Rows `row_indices` of the packed (n_rows, row_bytes) matrix, dequantized bit-exactly

@@ -71,3 +71,22 @@ def test_hip_dequantizer_interface(gpu) -> None:
     w = S.packed_weight(D.Q8_0, 4, 256, seed=1)
     got = host(HipDequantizer.dequantize(torch.from_numpy(w).cuda().reshape(-1, 34), D.Q8_0))
     assert np.array_equal(bits(got), bits(D.dequantize(D.Q8_0, w)))
+
+
+@pytest.mark.parametrize("ggml_type", [D.Q8_0, D.Q4_K, D.Q6_K, D.IQ4_XS])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_embedding_ids_and_dtypes(gpu, ggml_type, dtype) -> None:
+    """Rows of an odd number of blocks, ids of other integer types and orders, negative and
+    out-of-range ids, every layer dtype: torch's cast of the oracle's float32 rows."""
+    vocab, dim = 77, 768
+    w = S.packed_weight(ggml_type, vocab, dim, seed=22)
+    emb = DevicePackedEmbedding(upload_packed(w, vocab, torch.device("cuda")), dim, ggml_type, dtype)
+    full = torch.from_numpy(D.dequantize_matrix(ggml_type, w, vocab, dim)).to(dtype)
+    ids = torch.tensor([[0, -1, 76, 5], [-77, 3, 3, 40]])
+    for given in (ids.cuda(), ids.to(torch.int32).cuda(), ids.cuda().T, ids):
+        got = emb(given).cpu()
+        assert got.shape == (*given.shape, dim) and got.dtype == dtype
+        assert torch.equal(got, full[given.cpu() % vocab])
+    got = emb(torch.tensor([77, -78, 2, 1 << 40, -(1 << 40)]).cuda()).cpu()
+    assert got[[0, 1, 3, 4]].isnan().all() and torch.equal(got[2], full[2])
+    assert emb(torch.empty(0, 3, dtype=torch.int64, device="cuda")).shape == (0, 3, dim)
