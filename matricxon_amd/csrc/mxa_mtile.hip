@@ -1,18 +1,7 @@
-// Matrix-core matmul on 16 x 16 tiles, Q4_K / Q6_K / Q8_0: up to 64 activation rows, and the grouped
-// MoE forms (more rows: mxa_ptile.hip).
-//
-// Tiling. A workgroup of WAVES waves owns 16 * NT consecutive weight rows per wave and 16 * MT
-// activation rows; grid.y walks the activation rows, so a weight block is read once per 16 * MT
-// activation rows and an activation chunk once per 16 * NT * WAVES weight rows. The Q8_K
-// activations (always pre-quantized in the workspace here) are staged in LDS per chunk of kCB
-// blocks, in two buffers: the next chunk is loaded into registers while the current one is
-// computed and written to the other buffer afterwards, so one barrier per chunk suffices (a
-// buffer is rewritten only after every wave has passed the barrier that ends its last use). Each
-// wave loads its rows' block two ahead while it computes the current one.
-//
-// Operands: the tile builders of mxa_tiles.hpp, with A (16 activation rows x 64 k) read from LDS.
-// The blocks are folded in order 0..nb-1, so the outputs equal the oracle and the decode kernels
-// bit for bit.
+// Matrix-core matmul on 16 x 16 tiles, Q4_K / Q6_K / Q8_0 (operands: mxa_tiles.hpp): the block-split batched
+// decode for shapes that the streaming kernels do not take, its grouped MoE form, and the choice of kernel
+// for up to 16 activation rows (more: mxa_ptile.hip). The blocks are folded in order 0..nb-1, so the outputs
+// equal the oracle and the decode kernels bit for bit.
 #include "mxa_kernels.hpp"
 #include "mxa_tiles.hpp"
 
@@ -20,192 +9,6 @@
 
 namespace mxa {
 namespace {
-
-constexpr int kCB = 2;                    // blocks per activation chunk
-constexpr int kQStride = kCB * QK + 16;   // LDS bytes per activation row (padding: distinct banks)
-constexpr int kBStride = kCB * 16 + 8;    // LDS halves per activation row of bsums
-
-
-// LDS bytes of one activation chunk buffer for 16 * MT rows: q8 | bsums (fp16) | d.
-template <int MT>
-constexpr int kMtBuf = ((16 * MT * kQStride + 16 * MT * kBStride * 2 + kCB * 16 * MT * 4) + 15) / 16 * 16;
-
-// Row-tiled body: MT activation tiles x NT weight tiles of 16 rows per wave, WAVES waves;
-// workgroup wg of n_wg along N, activation tile group mg (rows 16 MT mg ..) of M rows.
-template <int TYPE, int MT, int NT, int WAVES>
-__device__ __forceinline__ void mtile_rows(const uint8_t* w, long long row_bytes, const Act& act,
-                                           YOut y, long long ldy, int M, int N, int wg, int n_wg,
-                                           int mg) {
-  using Tile = typename TileOf<TYPE>::T;
-  using W = typename Tile::W;
-  constexpr int kRows = 16 * MT;
-  constexpr int kThreads = 64 * WAVES;
-  extern __shared__ __align__(16) uint8_t smem[];  // two chunk buffers of kMtBuf<MT> bytes
-  auto aq = [&](int buf) { return (int8_t*)(smem + buf * kMtBuf<MT>); };
-  auto ab = [&](int buf) { return (_Float16*)(smem + buf * kMtBuf<MT> + kRows * kQStride); };
-  auto ad = [&](int buf) { return (float*)(smem + buf * kMtBuf<MT> + kRows * kQStride + kRows * kBStride * 2); };
-
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int ln = lane & 15, g = lane >> 4;
-  const int n0 = xcd_tile(wg, n_wg) * WAVES * 16 * NT + 16 * NT * wave;
-  const int m0 = mg * kRows;
-  const uint8_t* row[NT];
-#pragma unroll
-  for (int nt = 0; nt < NT; ++nt) row[nt] = w + (size_t)min(n0 + 16 * nt + ln, N - 1) * row_bytes;
-  const int nb = act.nb;
-  float acc[MT][NT][4];
-#pragma unroll
-  for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) acc[mt][nt][i] = 0.0f;
-
-  // weight blocks two ahead of the one computed (one ahead measured 4-6% slower: a block's
-  // compute does not cover the load latency; three ahead no faster)
-  W cur[NT], nxt[NT], nx2[NT];
-#pragma unroll
-  for (int nt = 0; nt < NT; ++nt) {
-    cur[nt] = Tile::load(row[nt], 0, g);
-    nxt[nt] = Tile::load(row[nt], min(1, nb - 1), g);
-  }
-
-  // Activation staging, software-pipelined: chunk c + 1 is loaded into registers while chunk c
-  // is computed, and written to LDS between the two barriers. Thread tid owns the same pieces of
-  // every chunk (rows >= M repeat row M - 1, blocks >= cn repeat the chunk's last block: those
-  // results are never stored).
-  constexpr int kQPieces = kRows * kCB * 16;                   // 16-byte pieces of q8
-  constexpr int kQPer = (kQPieces + kThreads - 1) / kThreads;
-  constexpr int kBPieces = kRows * kCB * 2;                    // halves of a block's 16 bsums
-  constexpr int kBPer = (kBPieces + kThreads - 1) / kThreads;
-  constexpr int kDPer = (kRows * kCB + kThreads - 1) / kThreads;
-  struct Stage {
-    u32x4a4 q[kQPer];
-    u32x4a4 b[kBPer];
-    float d[kDPer];
-  };
-  auto load_stage = [&](int c0) {
-    Stage st;
-    const int cn = min(kCB, nb - c0);
-#pragma unroll
-    for (int j = 0; j < kQPer; ++j) {
-      const int p = min(tid + kThreads * j, kQPieces - 1);
-      const int r = p / (kCB * 16), o = p - r * (kCB * 16), bb = min(o >> 4, cn - 1), pc = o & 15;
-      st.q[j] = ld16((const uint8_t*)(act.q + (size_t)min(m0 + r, M - 1) * act.k + (size_t)(c0 + bb) * QK) + 16 * pc);
-    }
-#pragma unroll
-    for (int j = 0; j < kBPer; ++j) {
-      const int p = min(tid + kThreads * j, kBPieces - 1);
-      const int r = p / (kCB * 2), o = p - r * (kCB * 2), bb = min(o >> 1, cn - 1), hf = o & 1;
-      st.b[j] = ld16((const uint8_t*)(act.bsums + ((size_t)min(m0 + r, M - 1) * nb + c0 + bb) * 16) + 16 * hf);
-    }
-#pragma unroll
-    for (int j = 0; j < kDPer; ++j) {
-      const int p = min(tid + kThreads * j, kRows * kCB - 1), bb = p / kRows, r = p - bb * kRows;
-      st.d[j] = act.d[(size_t)min(m0 + r, M - 1) * nb + c0 + min(bb, cn - 1)];
-    }
-    return st;
-  };
-  auto store_stage = [&](const Stage& st, int buf) {
-    int8_t* Aq = aq(buf);
-    _Float16* Ab = ab(buf);
-    float* Ad = ad(buf);
-#pragma unroll
-    for (int j = 0; j < kQPer; ++j) {
-      const int p = tid + kThreads * j;
-      if (p < kQPieces) {
-        const int r = p / (kCB * 16), o = p - r * (kCB * 16);
-        *(u32x4a4*)(Aq + r * kQStride + (o >> 4) * QK + 16 * (o & 15)) = st.q[j];
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < kBPer; ++j) {
-      const int p = tid + kThreads * j;
-      if (p < kBPieces) {  // bsums as fp16 (exact: |.| <= 2032)
-        const int r = p / (kCB * 2), o = p - r * (kCB * 2);
-        const uint32_t wv[4] = {st.b[j].x, st.b[j].y, st.b[j].z, st.b[j].w};
-        f16x8 hv;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          hv[2 * i] = (_Float16)(float)(int16_t)(wv[i] & 0xFFFFu);
-          hv[2 * i + 1] = (_Float16)(float)(int16_t)(wv[i] >> 16);
-        }
-        *(f16x8*)(Ab + r * kBStride + (o >> 1) * 16 + 8 * (o & 1)) = hv;
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < kDPer; ++j) {
-      const int p = tid + kThreads * j;
-      if (p < kRows * kCB) Ad[p] = st.d[j];
-    }
-  };
-
-  {
-    const Stage st0 = load_stage(0);
-    store_stage(st0, 0);
-  }
-  __syncthreads();
-  for (int c0 = 0; c0 < nb; c0 += kCB) {
-    const int cn = min(kCB, nb - c0), buf = (c0 / kCB) & 1;
-    const bool more = c0 + kCB < nb;
-    Stage st;
-    if (more) st = load_stage(c0 + kCB);
-    // the chunk's blocks in order; the next block's weights load meanwhile
-    const ActTile A{aq(buf), ab(buf), kQStride, kBStride};
-    const float* Ad = ad(buf);
-#pragma unroll
-    for (int i = 0; i < kCB; ++i) {
-      if (i < cn) {
-        const int b = c0 + i;
-        if (b + 2 < nb) {
-#pragma unroll
-          for (int nt = 0; nt < NT; ++nt) nx2[nt] = Tile::load(row[nt], b + 2, g);
-        }
-        typename Tile::P pp[NT];
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt) pp[nt] = Tile::prep(cur[nt], g);
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt) {
-          const typename Tile::F f = Tile::frag(A, i, mt, ln, g);
-#pragma unroll
-          for (int nt = 0; nt < NT; ++nt)
-            Tile::value(pp[nt], f, g, [&](int e, float v, float dd) {
-              acc[mt][nt][e] = Tile::fold(acc[mt][nt][e], Ad[i * kRows + 16 * mt + 4 * g + e], v, dd);
-            });
-          // no scheduling barrier between tiles: the compiler overlaps one tile's fold with the
-          // next tile's A reads and MFMAs (222 VGPRs at MT = 8, no spills; measured 7% faster at
-          // M = 512 and 6% at M = 2048 than one tile at a time)
-        }
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt) {
-          cur[nt] = nxt[nt];
-          nxt[nt] = nx2[nt];
-        }
-      }
-    }
-    if (more) store_stage(st, buf ^ 1);
-    __syncthreads();  // the next chunk is in LDS; every wave is done with this one
-  }
-#pragma unroll
-  for (int nt = 0; nt < NT; ++nt) {
-    const int n = n0 + 16 * nt + ln;
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int m = m0 + 16 * mt + 4 * g + i;
-        if (m < M && n < N) y.put((size_t)m * ldy + n, acc[mt][nt][i]);
-      }
-  }
-}
-
-template <int TYPE, int MT, int NT, int WAVES>
-__global__ __launch_bounds__(64 * WAVES) void mtile_kernel(const uint8_t* w, long long row_bytes, Act act,
-                                                           YOut y, long long ldy, int M,
-                                                           int N) {
-  mtile_rows<TYPE, MT, NT, WAVES>(w, row_bytes, act, y, ldy, M, N, blockIdx.x, gridDim.x,
-                                  blockIdx.y);
-}
 
 // Batched decode (M <= 16): 32 weight rows per workgroup and the blocks of each chunk split over
 // the 4 waves (wave w takes blocks w and w + 4 of an 8-block chunk, for both 16-row tiles), so that
@@ -370,23 +173,9 @@ __global__ __launch_bounds__(256, 2) void moe_dec_kernel(const uint8_t* w, long 
   }
 }
 
-template <int TYPE, int MT, int NT, int WAVES>
-int launch_mt(const uint8_t* w, long long row_bytes, const Act& act, YOut y, long long ldy, int M,
-              int N, hipStream_t stream) {
-  constexpr int kLds = 2 * kMtBuf<MT>;
-  allow_lds((const void*)mtile_kernel<TYPE, MT, NT, WAVES>, kLds);
-  const int rows = WAVES * 16 * NT;
-  const dim3 grid((N + rows - 1) / rows, (M + 16 * MT - 1) / (16 * MT));
-  hipLaunchKernelGGL((mtile_kernel<TYPE, MT, NT, WAVES>), grid, dim3(64 * WAVES), kLds, stream, w,
-                     row_bytes, act, y, ldy, M, N);
-  return 0;
-}
-
 template <int TYPE>
 int launch_mt_type(const uint8_t* w, long long row_bytes, const Act& act, YOut y, long long ldy,
                    int M, int N, hipStream_t stream) {
-  // M <= 16: the streaming kernel, else the block-split kernel unless the 64-row tiles alone give
-  // >= 512 workgroups
   // M <= 16: the per-wave streaming kernel where its slots fit LDS (measured on MI355X at M = 16,
   // the same bits: Q4_K 4096 x 4096 5.7 vs 7.1 us, 1024 x 4096 5.4 vs 6.3, Q8_0 4096 x 4096 7.1 vs
   // 8.4; Q4_K 14336 x 4096 12.1 vs 12.0-12.3), then the copy-wave kernels
@@ -394,14 +183,12 @@ int launch_mt_type(const uint8_t* w, long long row_bytes, const Act& act, YOut y
   if (M <= 16 && launch_bflow(TYPE, w, row_bytes, act, y, ldy, M, N, stream) == 0) return 0;
   if (M <= 16 && launch_bres(TYPE, w, row_bytes, act, y, ldy, M, N, stream) == 0) return 0;
   if (M <= 16 && launch_bstream(TYPE, w, row_bytes, act, y, ldy, M, N, stream) == 0) return 0;
-  if (M <= 16 && N < 512 * 64) {
+  if (M <= 16 && N < 512 * 64) {  // enough rows to fill the chip take the prefill tiles
     constexpr int RT = TYPE == T_Q6_K ? 1 : 2;
     const int tiles = (N + 16 * RT - 1) / (16 * RT);
     hipLaunchKernelGGL((mdec_kernel<TYPE, RT>), dim3(tiles), dim3(256), 0, stream, w, row_bytes, act, y, ldy, M, N);
     return 0;
   }
-  // up to 64 rows: 16-row activation tiles and 64 weight rows per workgroup; prefill: 32 x 32 tiles
-  if (M <= 64) return launch_mt<TYPE, 1, 1, 4>(w, row_bytes, act, y, ldy, M, N, stream);
   return launch_ptile(TYPE, w, row_bytes, act, y, ldy, M, N, stream);
 }
 

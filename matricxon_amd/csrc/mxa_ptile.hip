@@ -38,6 +38,7 @@ namespace {
 
 typedef int32_t i32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef int16_t i16x8 __attribute__((ext_vector_type(8)));
 
 __device__ __forceinline__ i32x16 mfma_i8(i32x4 a, i32x4 b, i32x16 c) {
   return __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, c, 0, 0, 0);
@@ -72,23 +73,32 @@ __device__ __forceinline__ V in_vgpr(V v) {
 
 __device__ __forceinline__ float as_f32(int v) { return __builtin_bit_cast(float, v); }
 
-// One block of the activations in LDS as a wave's tile mt reads it.
+// One block of the activations in LDS as a wave's tile mt reads it; the bsums as int16 (kRaw) or as fp16,
+// exactly (|bsum| <= 2032).
+template <bool kRaw>
 struct PAct {
   const uint8_t* q;    // swizzled rows of 256 bytes
-  const uint8_t* bs;   // bsums as fp16, 32 bytes per row
+  const uint8_t* bs;   // bsums, 32 bytes per row
   const float* d;
   int r, h;            // lane % 32, lane / 32
   __device__ __forceinline__ i32x4 a(int mt, int t) const {
     return __builtin_bit_cast(i32x4, *(const u32x4*)(q + (32 * mt + r) * QK + 16 * ((2 * t + h) ^ (r & 15))));
   }
-  __device__ __forceinline__ f16x8 b(int mt) const { return *(const f16x8*)(bs + (32 * mt + r) * 32 + 16 * h); }
+  // bsums 8 h .. 8 h + 7 of row r
+  __device__ __forceinline__ f16x8 b(int mt) const {
+    const uint8_t* p = bs + (32 * mt + r) * 32 + 16 * h;
+    if constexpr (kRaw)
+      return __builtin_convertvector(*(const i16x8*)p, f16x8);
+    else
+      return *(const f16x8*)p;
+  }
   // scales of activation rows 8 q4 + 4 h + 0..3 of tile mt
   __device__ __forceinline__ f32x4 xd(int mt, int q4) const { return *(const f32x4*)(d + 32 * mt + 8 * q4 + 4 * h); }
 };
 
 // The two-plane types' block, chunk by chunk.
-template <class T, int MTW>
-__device__ __forceinline__ void two_planes(const typename T::W& w, const PAct& A, const i32x16& magic, f32x16* acc) {
+template <class T, int MTW, class Act, class Sink>
+__device__ __forceinline__ void two_planes(const typename T::W& w, const Act& A, const i32x16& magic, Sink&& sink) {
   const typename T::S s = T::scales(w);
   const uint32_t m4 = in_vgpr(0x0F0F0F0Fu);
   i32x16 hi[MTW], lo[MTW];
@@ -107,13 +117,14 @@ __device__ __forceinline__ void two_planes(const typename T::W& w, const PAct& A
   }
   const typename T::F f = T::folds(w, s, A.h);
 #pragma unroll
-  for (int mt = 0; mt < MTW; ++mt) T::fold(f, A, mt, hi[mt], lo[mt], acc[mt]);
+  for (int mt = 0; mt < MTW; ++mt) sink(mt, T::value(f, A, mt, hi[mt], lo[mt]), f.d);
 }
 
 // Every type: W, a lane's bytes of one block of its weight row; load(lds, off, h), from the wave's
-// slot; and block<MTW>, which folds the block into the outputs of the wave's tiles.
+// slot; and block<MTW>, which calls sink(mt, v, d) with the block's 16 values of each tile and its
+// weight scale. The oracle's fold is acc = fma(xd, v, acc), or fma(xd * d, v, acc) where kScaled.
 struct PQ4 {
-  static constexpr bool kBsums = true;
+  static constexpr bool kBsums = true, kScaled = false;
   struct W {
     u32x4a4 hdr, q[4];
   };
@@ -155,28 +166,26 @@ struct PQ4 {
     f.k9 = in_vgpr(-9.0f * kMagicF);
     return f;
   }
-  __device__ __forceinline__ static void fold(const F& f, const PAct& A, int mt, const i32x16& hi,
-                                              const i32x16& lo, f32x16& acc) {
+  template <class Act>
+  __device__ __forceinline__ static f32x16 value(const F& f, const Act& A, int mt, const i32x16& hi,
+                                                 const i32x16& lo) {
     const f32x16 summ = __builtin_amdgcn_mfma_f32_32x32x16_f16(A.b(mt), f.bm, kZeroF, 0, 0, 0);
+    f32x16 v;
 #pragma unroll
-    for (int q4 = 0; q4 < 4; ++q4) {
-      const f32x4 xd = A.xd(mt, q4);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int i = 4 * q4 + e;
-        const float sumi = fmaf(as_f32(hi[i]), 8.0f, f.k9) + as_f32(lo[i]);
-        acc[i] = fmaf(xd[e], fmaf(f.d, sumi, -(f.dmin * summ[i])), acc[i]);
-      }
+    for (int i = 0; i < 16; ++i) {
+      const float sumi = fmaf(as_f32(hi[i]), 8.0f, f.k9) + as_f32(lo[i]);
+      v[i] = fmaf(f.d, sumi, -(f.dmin * summ[i]));
     }
+    return v;
   }
-  template <int MTW>
-  __device__ __forceinline__ static void block(const W& w, const PAct& A, const i32x16& magic, f32x16* acc) {
-    two_planes<PQ4, MTW>(w, A, magic, acc);
+  template <int MTW, class Act, class Sink>
+  __device__ __forceinline__ static void block(const W& w, const Act& A, const i32x16& magic, Sink&& sink) {
+    two_planes<PQ4, MTW>(w, A, magic, sink);
   }
 };
 
 struct PQ6 {
-  static constexpr bool kBsums = false;
+  static constexpr bool kBsums = false, kScaled = true;
   struct W {
     u32x4a4 ql[4], qh[2], sc;  // ql[64 hh + 32 q + 16 h ..] at 2 hh + q, qh[32 hh + 16 h ..]
     uint32_t d;
@@ -236,27 +245,21 @@ struct PQ6 {
   __device__ __forceinline__ static F folds(const W& w, const S&, int) {
     return F{in_vgpr(half_to_float(w.d)), in_vgpr(-257.0f * kMagicF)};
   }
-  __device__ __forceinline__ static void fold(const F& f, const PAct& A, int mt, const i32x16& hi,
-                                              const i32x16& lo, f32x16& acc) {
+  template <class Act>
+  __device__ __forceinline__ static f32x16 value(const F& f, const Act&, int, const i32x16& hi, const i32x16& lo) {
+    f32x16 v;
 #pragma unroll
-    for (int q4 = 0; q4 < 4; ++q4) {
-      const f32x4 xd = A.xd(mt, q4);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int i = 4 * q4 + e;
-        const float sumi = fmaf(as_f32(hi[i]), 256.0f, f.k257) + as_f32(lo[i]);
-        acc[i] = fmaf(xd[e] * f.d, sumi, acc[i]);
-      }
-    }
+    for (int i = 0; i < 16; ++i) v[i] = fmaf(as_f32(hi[i]), 256.0f, f.k257) + as_f32(lo[i]);
+    return v;
   }
-  template <int MTW>
-  __device__ __forceinline__ static void block(const W& w, const PAct& A, const i32x16& magic, f32x16* acc) {
-    two_planes<PQ6, MTW>(w, A, magic, acc);
+  template <int MTW, class Act, class Sink>
+  __device__ __forceinline__ static void block(const W& w, const Act& A, const i32x16& magic, Sink&& sink) {
+    two_planes<PQ6, MTW>(w, A, magic, sink);
   }
 };
 
 struct PQ8 {
-  static constexpr bool kBsums = false;
+  static constexpr bool kBsums = false, kScaled = false;
   struct W {
     // blocks 2 j and 2 j + 1 are 68 bytes from 68 j: d, 32 quants, d, 32 quants; this lane's half
     // of the even one's quants starts in the upper half of dword 4 h, the odd one's at dword 9 + 4 h
@@ -276,8 +279,8 @@ struct PQ8 {
     }
     return w;
   }
-  template <int MTW>
-  __device__ __forceinline__ static void block(const W& w, const PAct& A, const i32x16& magic, f32x16* acc) {
+  template <int MTW, class Act, class Sink>
+  __device__ __forceinline__ static void block(const W& w, const Act& A, const i32x16& magic, Sink&& sink) {
     const float kb = in_vgpr(kMagicF);
     i32x4 bq[8];
     float dk[8];
@@ -306,12 +309,7 @@ struct PQ8 {
         for (int i = 0; i < 16; ++i) bs[i] = fmaf(dk[k], as_f32(p[i]) - kb, bs[i]);
         asm("" : "+v"(bs));
       }
-#pragma unroll
-      for (int q4 = 0; q4 < 4; ++q4) {
-        const f32x4 xd = A.xd(mt, q4);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) acc[mt][4 * q4 + e] = fmaf(xd[e], bs[4 * q4 + e], acc[mt][4 * q4 + e]);
-      }
+      sink(mt, bs, 1.0f);
       __builtin_amdgcn_sched_barrier(0);
     }
   }
@@ -333,6 +331,51 @@ __host__ __device__ constexpr int ppieces(bool aligned) {
 }
 constexpr int pslot_bytes(int pieces) { return (32 * pieces + 63) / 64 * 1024; }
 
+__device__ __forceinline__ uint32_t uniform(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
+
+// 4 bytes per lane from `g` to LDS byte address lds + 4 * lane.
+__device__ __forceinline__ void copy4_to_lds(const void* g, uint32_t lds) {
+  asm volatile("global_load_lds_dword %0, off" ::"v"(g), "{m0}"(lds) : "memory");
+}
+
+// A wave's 32 weight rows, copied block by block into a slot that only it reads. Piece c of row q comes
+// from the 16-byte boundary at or below the block's start, so every piece holds at least one byte of the
+// block and none lies outside the 16-byte units that the matrix occupies. Rows >= N repeat row N - 1.
+template <class T>
+struct PWeights {
+  static constexpr int kMax = (32 * ppieces<T>(false) + 63) / 64;
+  const uint8_t* row0;  // the 16-byte boundary at or below the first row
+  uint32_t off[kMax], pc[kMax];
+  uint32_t mine;  // of lane % 32's row from row0
+  int pieces, copies;
+  __device__ __forceinline__ PWeights(const uint8_t* w, long long row_bytes, int n0, int N, int pieces_, int lane)
+      : pieces(pieces_), copies(pslot_bytes(pieces_) >> 10) {
+    const uint32_t mis = (uint32_t)((uintptr_t)w & 15);
+    const long long first = (long long)min(n0, N - 1) * row_bytes;
+    row0 = (const uint8_t*)((uintptr_t)w & ~(uintptr_t)15) + (first & ~15LL);
+    auto row_off = [&](int q) {
+      return mis + (uint32_t)(first & 15) + (uint32_t)((min(n0 + q, N - 1) - min(n0, N - 1)) * row_bytes);
+    };
+#pragma unroll
+    for (int i = 0; i < kMax; ++i) {
+      const int s = min(64 * i + lane, 32 * pieces - 1), q = s / pieces;
+      pc[i] = 16 * (uint32_t)(s - q * pieces);
+      off[i] = row_off(q);
+    }
+    mine = row_off(lane & 31);
+  }
+  __device__ __forceinline__ void copy(int b, uint32_t slot) const {
+#pragma unroll
+    for (int i = 0; i < kMax; ++i)
+      if (i < copies)
+        copy16_to_lds_s(row0, ((off[i] + (uint32_t)(T::kBytes * b)) & ~15u) + pc[i], uniform(slot + 1024 * i));
+  }
+  // where in the slot row r's block b starts
+  __device__ __forceinline__ int at(int b, int r) const {
+    return r * pieces * 16 + (int)((mine + (uint32_t)(T::kBytes * b)) & 15u);
+  }
+};
+
 // The outputs of activation rows m0 .. m0 + 32 MTW - 1 of M.
 template <int TYPE, int WN, int MTW>
 __device__ __forceinline__ void ptile_rows(const uint8_t* w, long long row_bytes, const Act& act, YOut y,
@@ -346,36 +389,9 @@ __device__ __forceinline__ void ptile_rows(const uint8_t* w, long long row_bytes
   const int n0 = (xcd_tile(wg, n_wg) * WN + wave) * 32, n = n0 + r;
   const int nb = act.nb;
 
-  // The wave's weights: piece c of row q is copied from the 16-byte boundary at or below the
-  // block's start, so every piece holds at least one byte of the block and none lies outside the
-  // 16-byte units that the matrix occupies. Only this wave reads its slot.
-  const uint8_t* wbase = (const uint8_t*)((uintptr_t)w & ~(uintptr_t)15);
-  const uint32_t mis = (uint32_t)((uintptr_t)w & 15);
+  const PWeights<T> pw(w, row_bytes, n0, N, pieces, lane);
   const int slot = 2 * kBuf + wave * pslot_bytes(pieces);
   const uint32_t slot0 = lds_addr(smem) + slot;
-  const long long row0 = (long long)min(n0, N - 1) * row_bytes;
-  constexpr int kWMax = (32 * ppieces<T>(false) + 63) / 64;
-  const int wcopies = (32 * pieces + 63) / 64;
-  uint32_t woff[kWMax], wpc[kWMax];
-#pragma unroll
-  for (int i = 0; i < kWMax; ++i) {
-    const int s = min(64 * i + lane, 32 * pieces - 1), q = s / pieces;
-    wpc[i] = 16 * (uint32_t)(s - q * pieces);
-    woff[i] = mis + (uint32_t)((min(n0 + q, N - 1) - min(n0, N - 1)) * row_bytes) + (uint32_t)(row0 & 15);
-  }
-  const uint8_t* wrow0 = wbase + (row0 & ~15LL);
-  const int my_piece0 = slot + r * pieces * 16;
-  const uint32_t my_off = mis + (uint32_t)((min(n, N - 1) - min(n0, N - 1)) * row_bytes) + (uint32_t)(row0 & 15);
-  auto copy_w = [&](int b) {
-#pragma unroll
-    for (int i = 0; i < kWMax; ++i)
-      if (i < wcopies)
-        copy16_to_lds_s(wrow0, ((woff[i] + (uint32_t)(T::kBytes * b)) & ~15u) + wpc[i],
-                        (uint32_t)__builtin_amdgcn_readfirstlane((int)(slot0 + 1024 * i)));
-  };
-  auto load_w = [&](int b) {
-    return T::load(smem, my_piece0 + (int)((my_off + (uint32_t)(T::kBytes * b)) & 15u), h);
-  };
 
   // this wave's copies of a block: 4 rows x 16 pieces each (rows >= M repeat row M - 1)
   constexpr int kCopies = kRows / 4 / WN;
@@ -419,13 +435,7 @@ __device__ __forceinline__ void ptile_rows(const uint8_t* w, long long row_bytes
       for (int j = 0; j < kBPer; ++j) {
         const int p = tid + kThreads * j;
         if (p < 2 * kRows) {
-          f16x8 hv;  // exact: |bsum| <= 2032
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            hv[2 * i] = (_Float16)(float)(int16_t)(sb[j][i] & 0xFFFFu);
-            hv[2 * i + 1] = (_Float16)(float)(int16_t)(sb[j][i] >> 16);
-          }
-          *(f16x8*)(bs + 16 * p) = hv;
+          *(f16x8*)(bs + 16 * p) = __builtin_convertvector(__builtin_bit_cast(i16x8, sb[j]), f16x8);
         }
       }
     }
@@ -444,23 +454,31 @@ __device__ __forceinline__ void ptile_rows(const uint8_t* w, long long row_bytes
   magic = in_vgpr(magic);
   load_s(0);
   copy_q(0, 0);
-  copy_w(0);
+  pw.copy(0, slot0);
   store_s(0);
   wait_vmcnt(0);
   __syncthreads();
   for (int b = 0; b < nb; ++b) {
     const int buf = b & 1;
     const bool more = b + 1 < nb;
-    const typename T::W cur = load_w(b);
+    const typename T::W cur = T::load(smem, slot + pw.at(b, r), h);
     if (more) {
       load_s(b + 1);
       copy_q(b + 1, buf ^ 1);
       wait_lgkm0();  // the weights are in registers: their slot takes the next block's
-      copy_w(b + 1);
+      pw.copy(b + 1, slot0);
     }
     const uint8_t* base = smem + buf * kBuf;
-    const PAct A{base, base + kRows * QK, (const float*)(base + kRows * (QK + 32)), r, h};
-    T::template block<MTW>(cur, A, magic, acc);
+    const PAct<false> A{base, base + kRows * QK, (const float*)(base + kRows * (QK + 32)), r, h};
+    T::template block<MTW>(cur, A, magic, [&](int mt, const f32x16& v, float d) {
+#pragma unroll
+      for (int q4 = 0; q4 < 4; ++q4) {
+        const f32x4 xd = A.xd(mt, q4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          acc[mt][4 * q4 + e] = fmaf(T::kScaled ? xd[e] * d : xd[e], v[4 * q4 + e], acc[mt][4 * q4 + e]);
+      }
+    });
     // the folds stay with their MFMAs (left alone, the compiler moves them past the next branch)
 #pragma unroll
     for (int mt = 0; mt < MTW; ++mt) asm volatile("" : "+v"(acc[mt]));
@@ -479,23 +497,12 @@ __device__ __forceinline__ void ptile_rows(const uint8_t* w, long long row_bytes
   }
 }
 
-// Two tiles per wave, or one where the second would have no row (the choice stands outside the block
-// loop: inside it, the accumulators' moves cost a tenth of the time).
-template <int TYPE, int WN, int MTW>
-__device__ __forceinline__ void ptile_any(const uint8_t* w, long long row_bytes, const Act& act, YOut y,
-                                          long long ldy, int M, int N, int pieces, int wg, int n_wg, int m0) {
-  if (MTW == 2 && m0 + 32 >= M)
-    ptile_rows<TYPE, WN, 1>(w, row_bytes, act, y, ldy, M, N, pieces, wg, n_wg, m0);
-  else
-    ptile_rows<TYPE, WN, MTW>(w, row_bytes, act, y, ldy, M, N, pieces, wg, n_wg, m0);
-}
-
 template <int TYPE, int WN, int MTW>
 __global__ __launch_bounds__(64 * WN, 2) void ptile_kernel(const uint8_t* w, long long row_bytes, Act act,
                                                            YOut y, long long ldy, int M, int N,
                                                            int pieces) {
-  ptile_any<TYPE, WN, MTW>(w, row_bytes, act, y, ldy, M, N, pieces, blockIdx.x, gridDim.x,
-                           32 * MTW * blockIdx.y);
+  ptile_rows<TYPE, WN, MTW>(w, row_bytes, act, y, ldy, M, N, pieces, blockIdx.x, gridDim.x,
+                            32 * MTW * blockIdx.y);
 }
 
 // Grouped MoE projection: item blockIdx.z of the (expert, chunk of 32 MTW rows) list
@@ -513,8 +520,116 @@ __global__ __launch_bounds__(64 * WN, 2) void moe_ptile_kernel(const uint8_t* w,
   a.q = act.q + (size_t)p0 * act.k;
   a.d = act.d + (size_t)p0 * act.nb;
   a.bsums = act.bsums + (size_t)p0 * act.nb * 16;
-  ptile_any<TYPE, WN, MTW>(w + (size_t)e * expert_stride, row_bytes, a, y.at((size_t)p0 * ldy), ldy, M, N,
-                           pieces, blockIdx.x, gridDim.x, 0);
+  const uint8_t* we = w + (size_t)e * expert_stride;
+  const YOut ye = y.at((size_t)p0 * ldy);
+  // an expert's last rows often need one tile only (the choice stands outside the block loop: inside it,
+  // the accumulators' moves cost a tenth of the time)
+  if (MTW == 2 && M <= 32)
+    ptile_rows<TYPE, WN, 1>(we, row_bytes, a, ye, ldy, M, N, pieces, blockIdx.x, gridDim.x, 0);
+  else
+    ptile_rows<TYPE, WN, MTW>(we, row_bytes, a, ye, ldy, M, N, pieces, blockIdx.x, gridDim.x, 0);
+}
+
+// Few tiles (short prompts, narrow matrices): the four waves of a workgroup share one tile of 32 weight
+// rows x 32 activation rows and take its blocks in turn, wave k blocks 4 r + k of round r, each with
+// its own copies of both operands. A round's block values meet in LDS, and wave j folds the outputs of
+// activation rows 8 j .. 8 j + 7 of each half, blocks in order, so the bits are the same.
+//
+// Bound: a wave alone on its SIMD takes about 1.1 us a block (one instruction per ~6 cycles, the copies'
+// latency), so what counts is the number of blocks in a row that one wave takes and the waves in
+// flight: two workgroups fit a CU (74 KB of LDS for Q4_K).
+constexpr int kKs = 4;
+template <class T>
+constexpr int ks_act_bytes() { return 32 * QK + (T::kBsums ? 1024 : 0) + 256; }
+constexpr int kKsV = 4096 + 256;  // a wave's block values, then its activation and weight scales
+
+template <int TYPE>
+__global__ __launch_bounds__(64 * kKs, 2) void ktile_kernel(const uint8_t* w, long long row_bytes, Act act,
+                                                            YOut y, long long ldy, int M, int N, int pieces) {
+  using T = typename PTileOf<TYPE>::T;
+  extern __shared__ __align__(16) uint8_t smem[];
+  const int lane = threadIdx.x & 63;
+  const int wave = (int)uniform(threadIdx.x >> 6);
+  const int r = lane & 31, h = lane >> 5;
+  const int n0 = xcd_tile(blockIdx.x, gridDim.x) * 32, n = n0 + r, m0 = 32 * blockIdx.y;
+  const int nb = act.nb;
+  const int slot = pslot_bytes(pieces);
+  const int mine = wave * (ks_act_bytes<T>() + slot), values = kKs * (ks_act_bytes<T>() + slot);
+  uint8_t* base = smem + mine;
+  const uint32_t lds0 = lds_addr(smem) + mine;
+  const PWeights<T> pw(w, row_bytes, n0, N, pieces, lane);
+
+  const int8_t* src[8];  // 4 activation rows per copy (rows >= M repeat row M - 1)
+#pragma unroll
+  for (int c = 0; c < 8; ++c) {
+    const int rr = 4 * c + (lane >> 4);
+    src[c] = act.q + (size_t)min(m0 + rr, M - 1) * act.k + 16 * ((lane & 15) ^ (rr & 15));
+  }
+  const float* dsrc = act.d + (size_t)min(m0 + r, M - 1) * nb;
+  const int16_t* bsrc = act.bsums + (size_t)min(m0 + (lane >> 1), M - 1) * nb * 16 + 8 * (lane & 1);
+  constexpr int kBs = 32 * QK, kD = kBs + (T::kBsums ? 1024 : 0), kW = kD + 256;
+  auto issue = [&](int b) {
+    pw.copy(b, lds0 + kW);
+#pragma unroll
+    for (int c = 0; c < 8; ++c) copy16_to_lds(src[c] + (size_t)b * QK, uniform(lds0 + 1024 * c));
+    if constexpr (T::kBsums) copy16_to_lds(bsrc + (size_t)b * 16, uniform(lds0 + kBs));
+    copy4_to_lds(dsrc + b, uniform(lds0 + kD));
+  };
+
+  i32x16 magic;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) magic[i] = kMagic;
+  magic = in_vgpr(magic);
+  f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+  if (wave < nb) issue(wave);
+  for (int b0 = 0; b0 < nb; b0 += kKs) {
+    const int b = b0 + wave;
+    if (b < nb) {
+      wait_vmcnt(0);
+      const typename T::W cur = T::load(base, kW + pw.at(b, r), h);
+      const PAct<true> A{base, base + kBs, (const float*)(base + kD), r, h};
+      f32x4* V = (f32x4*)(smem + values + wave * kKsV);
+      T::template block<1>(cur, A, magic, [&](int, const f32x16& v, float d) {
+#pragma unroll
+        for (int q4 = 0; q4 < 4; ++q4) V[64 * q4 + lane] = f32x4{v[4 * q4], v[4 * q4 + 1], v[4 * q4 + 2], v[4 * q4 + 3]};
+        // lanes of h = 0 keep the activation scales, those of h = 1 the weight scales
+        ((float*)(V + 256))[lane] = h ? d : A.d[r];
+      });
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this wave has read its operands
+      if (b + kKs < nb) issue(b + kKs);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kKs; ++k)
+      if (b0 + k < nb) {
+        const f32x4* V = (const f32x4*)(smem + values + k * kKsV);
+        const float* s = (const float*)(V + 256);
+        const f32x4 v = V[64 * wave + lane], xd = *(const f32x4*)(s + 8 * wave + 4 * h);
+        const float d = s[32 + r];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[e] = fmaf(T::kScaled ? xd[e] * d : xd[e], v[e], acc[e]);
+      }
+    __syncthreads();  // the values have been read
+  }
+  if (n < N) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int m = m0 + 8 * wave + 4 * h + e;
+      if (m < M) y.put((size_t)m * ldy + n, acc[e]);
+    }
+  }
+}
+
+template <int TYPE>
+int launch_k(const uint8_t* w, long long row_bytes, const Act& act, YOut y, long long ldy, int M, int N,
+             hipStream_t stream) {
+  using T = typename PTileOf<TYPE>::T;
+  const int pieces = ppieces<T>(((uintptr_t)w & 15) == 0 && row_bytes % 16 == 0);
+  const int lds = kKs * (ks_act_bytes<T>() + pslot_bytes(pieces) + kKsV);
+  allow_lds((const void*)ktile_kernel<TYPE>, lds);
+  hipLaunchKernelGGL((ktile_kernel<TYPE>), dim3((N + 31) / 32, (M + 31) / 32), dim3(64 * kKs), lds, stream, w,
+                     row_bytes, act, y, ldy, M, N, pieces);
+  return 0;
 }
 
 template <int TYPE, int WN, int MTW>
@@ -530,15 +645,22 @@ int launch_p(const uint8_t* w, long long row_bytes, const Act& act, YOut y, long
   return 0;
 }
 
-// Waves along the weight rows and activation tiles per wave. Two tiles share a wave's decoded weights,
-// eight waves an activation block in LDS, as long as the grid still fills the chip: measured on
-// MI355X (us, kernel alone, 8 x 2 / 4 x 2 / 2 x 1 waves x tiles): Q4_K 14336 x 4096 M = 2048
-// 326 / 336 / 446, 4096 x 4096 M = 1024 46.0 / 47.7 / 69, M = 128 41 / 28 / 20; Q6_K 4096 x 14336
-// M = 1024 239 / 247 / 443; Q8_0 4096 x 4096 M = 2048 114 / 111 / 157, M = 333 56 / 45 / 36.
+// Few 32 x 32 tiles take a workgroup each. Otherwise two activation tiles share a wave's decoded
+// weights, and eight waves an activation block in LDS, as long as the grid still fills the chip.
+// Measured on MI355X, us, kernel alone; workgroup per tile / two waves of one tile / four of two:
+//   Q4_K 4096 x 4096 M = 32 / 128 / 200 / 333 (128 / 512 / 896 / 1408 tiles) 9.8 / 20 / 28, 12.6 / 20 / 28,
+//   21 / 28 / 29, 31 / 34 / 30; 14336 x 4096 M = 64 / 128 (896 / 1792) 23 / 29 / 29, 40 / 34 / 30; Q6_K
+//   4096 x 14336 M = 256 (1024) 117 / 165 / -; Q8_0 4096 x 4096 M = 128 / 333 (512 / 1408) 23 / 27 / 43,
+//   62 / 36 / 45, 14336 x 4096 M = 48 (896; its workgroup per tile has a CU to itself) 49 / 32 / -;
+// eight waves of two tiles / four of two / two of one: Q4_K 14336 x 4096 M = 2048 326 / 336 / 446, 4096 x
+//   4096 M = 1024 46.0 / 47.7 / 69; Q6_K 4096 x 14336 M = 1024 239 / 247 / 443; Q8_0 4096 x 4096 M = 2048
+//   114 / 111 / 157.
 template <int TYPE>
 int launch_p_type(const uint8_t* w, long long row_bytes, const Act& act, YOut y, long long ldy, int M, int N,
                   hipStream_t stream) {
   const long long m_tiles = (M + 63) / 64, cus = cu_count();
+  const long long tiles = (long long)((N + 31) / 32) * ((M + 31) / 32);
+  if (tiles <= (TYPE == T_Q8_0 ? 2 : 4) * cus) return launch_k<TYPE>(w, row_bytes, act, y, ldy, M, N, stream);
   if (TYPE != T_Q8_0 && (N + 255) / 256 * m_tiles >= cus)
     return launch_p<TYPE, 8, 2>(w, row_bytes, act, y, ldy, M, N, stream);
   if ((N + 127) / 128 * m_tiles >= (TYPE == T_Q8_0 ? cus * 3 / 2 : cus * 3 / 4))

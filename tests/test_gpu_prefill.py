@@ -30,8 +30,9 @@ def check(gpu, oracle, t, w, x, n, k, shift=0):
 @pytest.mark.parametrize("t", TYPES)
 @pytest.mark.parametrize("n,k,m", [
     (1, 256, 65), (31, 256, 96), (33, 512, 97), (64, 768, 128), (129, 1280, 129), (257, 2816, 200),
-    (1000, 1024, 333),   # two waves, one tile
-    (8200, 256, 210),    # four waves, two tiles
+    (1, 256, 17), (33, 512, 32), (70, 768, 33), (129, 1280, 40), (32, 2816, 64),  # a workgroup per tile
+    (1000, 512, 1100),   # two waves, one tile
+    (8200, 256, 400),    # four waves, two tiles
     (16500, 512, 300),   # eight waves, two tiles
 ])
 def test_prefill_tiles_match_oracle(gpu, oracle, t, n, k, m) -> None:
@@ -41,9 +42,11 @@ def test_prefill_tiles_match_oracle(gpu, oracle, t, n, k, m) -> None:
 
 @pytest.mark.parametrize("t", TYPES)
 @pytest.mark.parametrize("shift", [4, 8, 12])
-def test_prefill_weight_alignment(gpu, oracle, t, shift) -> None:
-    w = S.packed_weight(t, 70, 1280, seed=9)
-    check(gpu, oracle, t, w, S.activations(70, 1280, seed=10), 70, 1280, shift)
+@pytest.mark.parametrize("m", [70, 1100])
+def test_prefill_weight_alignment(gpu, oracle, t, shift, m) -> None:
+    n = 70 if m == 70 else 1000  # a workgroup per tile, waves of tiles
+    w = S.packed_weight(t, n, 1280, seed=9)
+    check(gpu, oracle, t, w, S.activations(m, 1280, seed=10), n, 1280, shift)
 
 
 @pytest.mark.parametrize("t", TYPES)
@@ -51,7 +54,7 @@ def test_prefill_weight_alignment(gpu, oracle, t, shift) -> None:
 def test_prefill_largest_sums(gpu, oracle, t, sign) -> None:
     """Every code, scale and activation at its largest magnitude, all products of one sign: the sums
     that the float conversion of the integer planes has to hold."""
-    n, k, m = 40, 512, 80
+    n, k, m = 40, 1536, 80
     w = S.packed_weight(t, n, k, seed=1).reshape(n, -1)
     if t == D.Q4_K:
         b = w.reshape(-1, 144)
