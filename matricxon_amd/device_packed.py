@@ -164,22 +164,23 @@ class DevicePackedLinear(nn.Module):
         if x.dtype != self._dtype:
             x = x.to(self._dtype)
         bf16 = self._dtype == torch.bfloat16  # the kernels read and write bfloat16 themselves
-        dev = self.packed.device
+        packed = self.packed
+        dev = packed.device
         n, big_n = x.numel() // k, self.out_features
         ws = HANDOFF.claim(x) if self._ggml_type != _IQ4_XS else None
         if ws is not None:  # x came from a fused producer that also wrote its Q8_K blocks
             y = torch.empty((n, big_n), dtype=torch.bfloat16 if bf16 else torch.float32, device=dev)
-            self._gemm.matmul_q8k(self._ggml_type, self.packed, ws, None, y, n, big_n, k)
+            self._gemm.matmul_q8k(self._ggml_type, packed, ws, None, y, n, big_n, k)
         elif bf16 and x.device == dev and n > 0:
-            xb = x.reshape(n, k)
+            xb = x if x.dim() == 2 else x.reshape(n, k)
             if not xb.is_contiguous() or xb.data_ptr() % 16 != 0:
                 xb = xb.clone(memory_format=torch.contiguous_format)
             y = torch.empty((n, big_n), dtype=torch.bfloat16, device=dev)
-            self._gemm._gemm_bf16(self._ggml_type, self.packed, xb, y, n, big_n, k)
+            self._gemm._gemm_bf16(self._ggml_type, packed, xb, y, n, big_n, k)
         elif bf16:
-            y = self._gemm.matmul_bf16(self._ggml_type, self.packed, x.reshape(-1, k), big_n, k)
+            y = self._gemm.matmul_bf16(self._ggml_type, packed, x.reshape(-1, k), big_n, k)
         else:
-            y = self._gemm.matmul(self._ggml_type, self.packed, x.reshape(-1, k), big_n, k)
+            y = self._gemm.matmul(self._ggml_type, packed, x.reshape(-1, k), big_n, k)
         return self.finish(y, lead)
 
     def _forward_f32(self, x2: torch.Tensor) -> torch.Tensor:
@@ -200,7 +201,8 @@ class DevicePackedLinear(nn.Module):
         in its dtype, plus bias."""
         if y.dtype != self._dtype:
             y = y.to(self._dtype)
-        y = y.reshape(*lead, self.out_features)
+        if len(lead) != 1:
+            y = y.reshape(*lead, self.out_features)
         return y if self.bias is None else y + self.bias
 
 

@@ -27,13 +27,13 @@ import threading
 import torch
 from torch import nn
 
-from matricxon_amd.gemm import HipGemm
+from matricxon_amd.gemm import HipGemm, _stream
 
 _IQ4_XS = 23
 
 
 def _stream_of(device: torch.device) -> int | None:
-    return torch.cuda.current_stream(device).cuda_stream if device.type == "cuda" else None
+    return _stream(device) if device.type == "cuda" else None
 
 
 class _Handoff:
@@ -62,7 +62,7 @@ class _Handoff:
         if slot is None or not x.is_contiguous():
             return None
         out, version, workspace, device, stream = slot
-        if (x.dtype != out.dtype or x.device != device or x.data_ptr() != out.data_ptr()
+        if (x.data_ptr() != out.data_ptr() or x.dtype != out.dtype or x.device != device
                 or x.numel() != out.numel()
                 or x.shape[-1] != out.shape[-1] or x._version != version
                 or out._version != version or _stream_of(device) != stream):
@@ -108,7 +108,8 @@ class HipFusedOps:
                 or (x.dtype == torch.bfloat16 and x.shape[-1] > _RMS_BF16_MAX)):
             return None
         out, ws = self._gemm.rms_norm_q8k(x, weight, eps)
-        out = out.view(x.shape)
+        if out.shape != x.shape:
+            out = out.view(x.shape)
         HANDOFF.offer(out, ws)
         return out
 
@@ -118,7 +119,8 @@ class HipFusedOps:
                 or gate.shape[-1] % 256 != 0 or gate.numel() == 0):
             return None
         out, ws = self._gemm.silu_mul_q8k(gate, up)
-        out = out.view(gate.shape)
+        if out.shape != gate.shape:
+            out = out.view(gate.shape)
         HANDOFF.offer(out, ws)
         return out
 
@@ -129,15 +131,20 @@ def project_shared(owner: nn.Module, names: tuple[str, ...], x: torch.Tensor) ->
     from matricxon_amd.device_packed import DevicePackedLinear
 
     mods = [getattr(owner, name) for name in names]
-    if (not 1 <= len(mods) <= 4 or x.device.type != "cuda"
-            or not all(isinstance(m, DevicePackedLinear) for m in mods)
-            or len({m.in_features for m in mods}) != 1 or len({m.dtype for m in mods}) != 1
-            or len({m.packed.device for m in mods}) != 1 or x.shape[-1] != mods[0].in_features):
+    # (type, packed, outputs) of a group of one input width, dtype and device; None for anything else
+    items = None
+    if 1 <= len(mods) <= 4 and x.device.type == "cuda" and \
+            all(isinstance(m, DevicePackedLinear) for m in mods):
+        k, dtype = mods[0].in_features, mods[0].dtype
+        items = [(m.ggml_type, m.packed, m.out_features) for m in mods]
+        device = items[0][1].device
+        if x.shape[-1] != k or any(m.in_features != k or m.dtype != dtype for m in mods) or \
+                any(p.device != device for _, p, _ in items):
+            items = None
+    if items is None:
         return [m(x) for m in mods]
-    dtype, k = mods[0].dtype, mods[0].in_features
     lead = x.shape[:-1]
-    xd = x.to(dtype)  # each module casts x to its dtype first (device_packed.py:54)
-    items = [(m.ggml_type, m.packed, m.out_features) for m in mods]
+    xd = x if x.dtype == dtype else x.to(dtype)  # each module casts x to its dtype (device_packed.py:54)
     gemm = HipGemm.get()
     bf16 = dtype == torch.bfloat16  # bfloat16 outputs straight from the kernels
     ws = HANDOFF.claim(xd)

@@ -9,6 +9,7 @@ the packed weight is a device uint8 tensor instead of an mmap'd memoryview, x an
 device, and the call is asynchronous on torch's current HIP stream (no host sync).
 """
 
+import ctypes
 import logging
 
 import torch
@@ -64,6 +65,20 @@ def _require_device_tensor(name: str, t: torch.Tensor) -> None:
         raise ValueError(f"{name} must be a tensor on a HIP device, got {getattr(t, 'device', t)}")
 
 
+def _rows16(t: torch.Tensor, k: int) -> torch.Tensor:
+    """`t` (..., k) as contiguous rows that start on a 16-byte boundary: itself where it is that."""
+    if t.is_contiguous() and t.data_ptr() % 16 == 0:
+        return t
+    return _aligned16(t.detach().reshape(-1, k).contiguous())
+
+
+def _weight_arrays(items: list[tuple[int, torch.Tensor, int]], outs: list[int]):
+    """The types, weight addresses and output widths of a group as the library's host arrays."""
+    n = len(items)
+    return ((ctypes.c_int * n)(*[int(t) for t, _, _ in items]),
+            (ctypes.c_void_p * n)(*[p.data_ptr() for _, p, _ in items]), (ctypes.c_int * n)(*outs))
+
+
 def _aligned16(t: torch.Tensor) -> torch.Tensor:
     """`t`, or a copy of it when its data does not start on a 16-byte boundary (the kernels read
     activations as 16-byte vectors; a view into the middle of a tensor may start anywhere)."""
@@ -103,6 +118,9 @@ class HipGemm:
 
     # -- capability queries ---------------------------------------------------------------------
     def supports(self, ggml_type: int, in_features: int) -> bool:
+        # `mxa_supports`' own rule, asked here first: a library call costs every projection 0.5 us
+        if in_features > 0 and in_features % 256 == 0 and ggml_type in GEOMETRY:
+            return True
         supported = bool(self._lib.mxa_supports(int(ggml_type), int(in_features)))
         if not supported and int(ggml_type) not in self._fallback_types_logged:
             self._fallback_types_logged.add(int(ggml_type))
@@ -155,11 +173,13 @@ class HipGemm:
     def _check_packed(self, ggml_type: int, packed: torch.Tensor, out_features: int,
                       in_features: int) -> None:
         _require_device_tensor("packed", packed)
-        expected = (out_features, self.row_bytes(ggml_type, in_features))
-        if packed.dtype != torch.uint8 or tuple(packed.shape) != expected:
+        block, size = GEOMETRY[ggml_type]
+        shape = packed.shape
+        if packed.dtype != torch.uint8 or len(shape) != 2 or shape[0] != out_features or \
+                shape[1] != in_features // block * size:
             raise ValueError(
-                f"packed must be uint8 {expected} for type {ggml_type}, got "
-                f"{packed.dtype} {tuple(packed.shape)}"
+                f"packed must be uint8 {(out_features, in_features // block * size)} for type "
+                f"{ggml_type}, got {packed.dtype} {tuple(shape)}"
             )
         if not packed.is_contiguous():
             raise ValueError("packed rows must be contiguous")
@@ -308,8 +328,6 @@ class HipGemm:
         `out`, if given, is the (n_tokens, sum of out_features) result buffer the outputs are
         views of. `bf16`: x taken as bfloat16 and the outputs bfloat16 (`mxa_gemm_multi_bf16`,
         a bfloat16 layer's projections)."""
-        import ctypes
-
         if not 1 <= len(items) <= 4:
             raise ValueError("matmul_multi takes 1 to 4 weights")
         in_features = x.shape[-1]
@@ -341,12 +359,9 @@ class HipGemm:
             need[is_iq4] = max(need[is_iq4], int(size_of(int(t), n_tokens, in_features)))
         ws_bytes = need[False] + need[True]
         ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=device)
-        n = len(items)
-        types = (ctypes.c_int * n)(*[int(t) for t, _, _ in items])
-        ptrs = (ctypes.c_void_p * n)(*[p.data_ptr() for _, p, _ in items])
-        couts = (ctypes.c_int * n)(*outs)
+        types, ptrs, couts = _weight_arrays(items, outs)
         fn = self._lib.mxa_gemm_multi_bf16 if bf16 else self._lib.mxa_gemm_multi
-        status = fn(n, types, ptrs, couts, xc.data_ptr(), y.data_ptr(), n_tokens, in_features,
+        status = fn(len(items), types, ptrs, couts, xc.data_ptr(), y.data_ptr(), n_tokens, in_features,
                     ws.data_ptr(), ws_bytes, _stream(device))
         self._check(status, "mxa_gemm_multi", int(items[0][0]))
         self._calls += 1
@@ -381,12 +396,14 @@ class HipGemm:
         for those dtypes (app/architectures/layers.py:77-81), out bfloat16 (M, K), and the Q8_K
         blocks of out. K up to 16384."""
         k = x.shape[-1]
-        xb = _aligned16(x.detach().reshape(-1, k).contiguous())
-        wb = _aligned16(weight.detach().to(x.device).contiguous())
-        m = xb.shape[0]
+        xb = _rows16(x, k)
+        wb = weight
+        if wb.device != x.device or not wb.is_contiguous() or wb.data_ptr() % 16 != 0:
+            wb = _aligned16(weight.detach().to(x.device).contiguous())
         if wb.shape != (k,):
             raise ValueError("weight must have shape (K,) for x (..., K)")
-        out = torch.empty_like(xb) if want_out else None
+        m = xb.numel() // k
+        out = torch.empty((m, k), dtype=torch.bfloat16, device=x.device) if want_out else None
         ws = torch.empty(q8k_bytes(m, k), dtype=torch.uint8, device=x.device)
         status = self._lib.mxa_rms_norm_q8_k_bf16(xb.data_ptr(), wb.data_ptr(), float(eps), m, k,
                                                   None if out is None else out.data_ptr(),
@@ -404,7 +421,8 @@ class HipGemm:
         if gate.shape != up.shape or gate.dim() == 0:
             raise ValueError("gate and up must have the same shape")
         k = gate.shape[-1]
-        g2, u2 = gate.detach().reshape(-1, k), up.detach().reshape(-1, k)
+        g2, u2 = (gate, up) if gate.dim() == 2 else \
+            (gate.detach().reshape(-1, k), up.detach().reshape(-1, k))
         if g2.dtype == u2.dtype == torch.bfloat16:
             return self._silu_mul_q8k_bf16(g2, u2, want_out)
         if not (g2.dtype == u2.dtype == torch.float32 and u2.device == g2.device
@@ -426,18 +444,19 @@ class HipGemm:
         """`silu_mul_q8k` of bfloat16 (M, K) gate and up (read in place when they share a row
         stride, a multiple of 4, with unit column stride and 8-byte aligned data, as the halves of a
         gate|up output): torch's steps for bfloat16 tensors, out bfloat16."""
-        k = g2.shape[-1]
-        if not (u2.device == g2.device and g2.stride(-1) == u2.stride(-1) == 1
-                and g2.stride(0) == u2.stride(0) and g2.stride(0) >= k and g2.stride(0) % 4 == 0
+        m, k = g2.shape
+        dev, (ld, step) = g2.device, g2.stride()
+        if not (u2.device == dev and u2.stride() == (ld, step) and step == 1
+                and ld >= k and ld % 4 == 0
                 and g2.data_ptr() % 8 == 0 and u2.data_ptr() % 8 == 0):
-            g2 = _aligned16(g2.contiguous())
-            u2 = _aligned16(u2.to(g2.device).contiguous())
-        m = g2.shape[0]
-        out = torch.empty((m, k), dtype=torch.bfloat16, device=g2.device) if want_out else None
-        ws = torch.empty(q8k_bytes(m, k), dtype=torch.uint8, device=g2.device)
-        status = self._lib.mxa_silu_mul_q8_k_bf16(g2.data_ptr(), u2.data_ptr(), g2.stride(0), m, k,
+            g2 = _aligned16(g2.detach().contiguous())
+            u2 = _aligned16(u2.detach().to(dev).contiguous())
+            ld = k
+        out = torch.empty((m, k), dtype=torch.bfloat16, device=dev) if want_out else None
+        ws = torch.empty(q8k_bytes(m, k), dtype=torch.uint8, device=dev)
+        status = self._lib.mxa_silu_mul_q8_k_bf16(g2.data_ptr(), u2.data_ptr(), ld, m, k,
                                                   None if out is None else out.data_ptr(),
-                                                  ws.data_ptr(), ws.numel(), _stream(g2.device))
+                                                  ws.data_ptr(), ws.numel(), _stream(dev))
         self._check(status, "mxa_silu_mul_q8_k_bf16", 15)
         return out, ws
 
@@ -621,8 +640,6 @@ class HipGemm:
         """`matmul_multi` on activations already quantized into `workspace` (by a fused producer
         or `quantize_into`); K-quant and Q8_0 weights only. Outputs float32, or bfloat16 (`dtype`,
         or `out`'s dtype) rounded as torch's cast."""
-        import ctypes
-
         if not 1 <= len(items) <= 4:
             raise ValueError("matmul_multi_q8k takes 1 to 4 weights")
         device = items[0][1].device
@@ -637,13 +654,10 @@ class HipGemm:
               or not out.is_contiguous() or tuple(out.shape) != (n_tokens, sum(outs))):
             raise ValueError("out must be a contiguous float32 or bfloat16 (n_tokens, sum of "
                              "out_features) tensor on the weights' device")
-        n = len(items)
-        types = (ctypes.c_int * n)(*[int(t) for t, _, _ in items])
-        ptrs = (ctypes.c_void_p * n)(*[p.data_ptr() for _, p, _ in items])
-        couts = (ctypes.c_int * n)(*outs)
+        types, ptrs, couts = _weight_arrays(items, outs)
         fn = self._lib.mxa_gemm_multi_q8k_bf16 if out.dtype == torch.bfloat16 else \
             self._lib.mxa_gemm_multi_q8k
-        status = fn(n, types, ptrs, couts, out.data_ptr(), n_tokens, in_features,
+        status = fn(len(items), types, ptrs, couts, out.data_ptr(), n_tokens, in_features,
                     workspace.data_ptr(), workspace.numel(), _stream(device))
         self._check(status, "mxa_gemm_multi_q8k", int(items[0][0]))
         self._calls += 1

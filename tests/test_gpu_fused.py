@@ -225,3 +225,27 @@ def test_project_shared_bf16_and_bias(gpu) -> None:
     ya, yb = project_shared(mods, ("a", "b"), x)
     assert ya.dtype == torch.bfloat16 and ya.shape == (2, 3, 64)
     assert torch.equal(ya, mods.a(x)) and torch.equal(yb, mods.b(x))
+
+
+def test_bf16_producers_on_views(gpu) -> None:
+    """bfloat16 operands that the launches do not read in place (a strided weight, rows that start off a
+    16-byte boundary, transposed or differently strided gate and up, three dimensions) give what their
+    contiguous copies give."""
+    import torch
+
+    k, g = 512, torch.Generator().manual_seed(3)
+    big = torch.randn(2 * 6 * k + 64, generator=g).to(torch.bfloat16).cuda()
+    wide = torch.randn(2 * k, generator=g).to(torch.bfloat16).cuda()
+    for x in (big[:6 * k].view(6, k), big[1:1 + 6 * k].view(6, k), big[:6 * k].view(2, 3, k),
+              big[:6 * k].view(k, 6).T, big[:12 * k].view(6, 2 * k)[:, k:]):
+        for w in (wide[:k], wide[::2], wide[1:1 + k]):
+            out, ws = gpu.rms_norm_q8k(x, w, 1e-5)
+            want, ws2 = gpu.rms_norm_q8k(x.reshape(-1, k).clone(), w.clone(), 1e-5)
+            assert torch.equal(out, want) and torch.equal(ws[:6 * k], ws2[:6 * k])
+    a, b = big[:6 * k].view(6, k), big[6 * k:12 * k].view(6, k)
+    halves = big[:12 * k].view(6, 2 * k)
+    for gate, up in ((a, b), (halves[:, :k], halves[:, k:]), (halves[:, :k], b), (a.view(k, 6).T, b),
+                     (big[1:1 + 6 * k].view(6, k), b), (a.view(2, 3, k), b.view(2, 3, k))):
+        out, ws = gpu.silu_mul_q8k(gate, up)
+        want, ws2 = gpu.silu_mul_q8k(gate.reshape(-1, k).clone(), up.reshape(-1, k).clone())
+        assert torch.equal(out, want) and torch.equal(ws[:6 * k], ws2[:6 * k])
