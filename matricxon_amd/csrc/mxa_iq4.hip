@@ -4,24 +4,22 @@
 // IQ4_NL grid, dl = d * (ls - 32) per 32-value sub-block). Here x is first split into two bf16
 // parts, x = hi + lo (hi = x rounded to bf16, lo = the rest rounded to bf16; relative error of the
 // pair about 2^-17), written to the workspace by split_bf16_kernel. The grid values are small
-// integers, exact in bf16, so v_mfma_f32_16x16x32_bf16 on (hi, K) then (lo, K) gives sum(K * x) of
-// one sub-block per MFMA pair: with A = x (16 activation rows x 32 k) and B = K (32 k x 16 weight
-// rows), lane l supplies row (l % 16) and k-group g = l / 16, i.e. elements 32 t + 8 g + (0..7) of
-// sub-block t. The sub-block scale dl is applied in fp32 after the MFMA. The result meets the
-// float tolerance against the reference (rel-L2 <= 1e-4); its summation order differs from the
+// integers, exact in bf16, so bf16 MFMAs on (hi, K) and (lo, K) give sum(K * x) of one sub-block.
+// The sub-block scale dl is applied in fp32 after them. The result meets the float tolerance against the reference (rel-L2 <= 1e-4); its summation order differs from the
 // decode kernels', which is why batches of up to 16 rows stay on those.
 #include "mxa_kernels.hpp"
+#include "mxa_pcopy.hpp"
 
 #pragma clang fp contract(off)
 
 namespace mxa {
 namespace {
 
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));  // 16-byte aligned
 
-constexpr int kXStride = QK * 2 + 16;      // LDS bytes per activation row (bf16), padded
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+constexpr f32x16 kZero16 = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
 
 // bf16 bits of x rounded to nearest even (NaN stays NaN, overflow gives +-Inf).
 __device__ __forceinline__ uint32_t bf16_rne(float x) {
@@ -62,148 +60,116 @@ __device__ __forceinline__ u32x4a4 grid_bf16x8(uint32_t a, uint32_t b) {
                  __builtin_amdgcn_perm(f[5], f[4], 0x07060302u), __builtin_amdgcn_perm(f[7], f[6], 0x07060302u)};
 }
 
-struct IQ4W {
-  uint32_t hdr[2];   // d | scales_h, scales_l
-  uint32_t qs[16];   // for sub-block t: qs[16 t + 8 (g & 1) ..] as two dwords
+// Tiling (as mxa_ptile.hip): a wave owns 32 weight rows x 32 MTW activation rows, a workgroup WN waves
+// along the weight rows. v_mfma_f32_32x32x16_bf16 takes 16 of a sub-block's 32 values: lane (row, h)
+// holds bytes 8 h .. 8 h + 7 of the sub-block's 16, whose low nibbles are elements 8 h .. of the first
+// step's 16 and whose high nibbles are those of the second's, so both operands come in natural order.
+// A sub-block is four MFMAs (two steps of hi, two of lo) into a sum of its own, scaled by dl in fp32.
+// The activations of half a block (128 values: 256 bytes of hi, 256 of lo per row) go straight into one of
+// two LDS buffers, piece c of row r at place c ^ (r & 15); a wave's weights into a slot that only it reads.
+//
+// Bound: instruction issue (a sub-block of 32 rows costs about 50 VALU instructions to look its 512
+// values up as bf16, 16 per activation tile to scale, four MFMAs of 32 cycles per tile). Measured on
+// MI355X against 16 x 16 tiles whose eight waves read every operand from LDS (us per call, the same bits):
+// 4096 x 4096 M = 512 58 vs 94, M = 2048 200 vs 283 (344 TFLOP/s), 14336 x 4096 M = 2048 632 vs 941,
+// 4096 x 14336 M = 128 129 vs 261.
+struct PIQ4 {
+  static constexpr int kBytes = 136, kShift = 8;  // blocks start at 8-byte multiples of the row
 };
 
-__device__ __forceinline__ IQ4W load_iq4(const uint8_t* row, int b, int g) {
-  const uint8_t* blk = row + (size_t)b * 136;  // 8-byte aligned blocks (4-byte aligned rows)
-  IQ4W L;
-  const u32x2a4 h = ld8(blk);
-  L.hdr[0] = h.x, L.hdr[1] = h.y;
-#pragma unroll
-  for (int t = 0; t < 8; ++t) {
-    const u32x2a4 v = ld8(blk + 8 + 16 * t + 8 * (g & 1));
-    L.qs[2 * t] = v.x, L.qs[2 * t + 1] = v.y;
-  }
-  return L;
-}
-
-// A workgroup takes 16 NT weight rows per wave (8 waves) x 16 MT activation rows. The activations
-// of a block (bf16 hi and lo, 2 x 512 B per row) go to one of two LDS buffers: the next block's
-// are loaded into registers while the current block is computed and written to the other buffer
-// afterwards, so one barrier per block suffices (a buffer is rewritten only after every wave has
-// passed the barrier that ends its last use). Per sub-block t the B operand is the grid values of
-// elements 32 t + 8 g .. of row n; one MFMA pair (hi, then lo) gives sum(K * x), scaled by dl in
-// fp32, sub-blocks and blocks in order. Every wave reads the workgroup's activation tiles from LDS,
-// so the NT weight tiles of a wave share each A-operand read (LDS bytes per MFMA / NT).
-constexpr int kIq4Waves = 8;
-
-template <int MT, int NT>
-__global__ __launch_bounds__(64 * kIq4Waves) void iq4_mtile_kernel(const uint8_t* w, long long row_bytes,
-                                                                   const uint16_t* __restrict__ xh,
-                                                                   const uint16_t* __restrict__ xl,
-                                                                   int K, YOut y,
-                                                                   long long ldy, int M, int N) {
-  constexpr int kRows = 16 * MT;
-  constexpr int kWgRows = 16 * NT * kIq4Waves;
-  constexpr int kBuf = 2 * kRows * kXStride;                  // hi rows, then lo rows
-  constexpr int kPieces = kRows * 64 / (64 * kIq4Waves);      // 16-byte pieces per thread
-  extern __shared__ __align__(16) uint8_t smem[];
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int ln = lane & 15, g = lane >> 4;
-  const int n0 = xcd_tile(blockIdx.x, gridDim.x) * kWgRows + 16 * NT * wave;
-  const int m0 = blockIdx.y * kRows;
-  const uint8_t* row[NT];
-#pragma unroll
-  for (int nt = 0; nt < NT; ++nt) row[nt] = w + (size_t)min(n0 + 16 * nt + ln, N - 1) * row_bytes;
+template <int WN, int MTW>
+__global__ __launch_bounds__(64 * WN, 2) void iq4_ptile_kernel(const uint8_t* w, long long row_bytes,
+                                                               const uint16_t* __restrict__ xh,
+                                                               const uint16_t* __restrict__ xl, int K, YOut y,
+                                                               long long ldy, int M, int N, int pieces) {
+  constexpr int kRows = 32 * MTW, kBuf = 2 * kRows * 256;
+  extern __shared__ __align__(16) uint8_t smem[];  // two activation buffers (hi rows, lo rows), the slots
+  const int lane = threadIdx.x & 63;
+  const int wave = (int)uniform(threadIdx.x >> 6);
+  const int r = lane & 31, h = lane >> 5;
+  const int n0 = (xcd_tile(blockIdx.x, gridDim.x) * WN + wave) * 32, n = n0 + r, m0 = kRows * blockIdx.y;
   const int nb = K / QK;
-  f32x4 acc[MT][NT];
-#pragma unroll
-  for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  const PWeights<PIQ4> pw(w, row_bytes, n0, N, pieces, lane);
+  const int slot = 2 * kBuf + wave * pslot_bytes(pieces);
+  const uint32_t lds0 = lds_addr(smem), slot0 = lds0 + slot;
 
-  // thread tid stages pieces p = tid + 512 i: row p / 64, hi (p % 64 < 32) or lo, piece p % 32;
-  // rows >= M repeat row M - 1
-  u32x4a4 stage[kPieces];
-  auto load_x = [&](int b) {
+  // this wave's copies of half a block: 4 rows of hi or lo each (rows >= M repeat row M - 1)
+  constexpr int kCopies = 2 * kRows / 4 / WN;
+  static_assert(kCopies * 4 * WN == 2 * kRows, "whole copies per wave");
+  const uint16_t* src[kCopies];
 #pragma unroll
-    for (int i = 0; i < kPieces; ++i) {
-      const int p = tid + 64 * kIq4Waves * i, r = p >> 6, pc = p & 63, part = pc >> 5, q = pc & 31;
-      const size_t src = (size_t)min(m0 + r, M - 1) * K + (size_t)b * QK;
-      stage[i] = ld16((const uint8_t*)((part ? xl : xh) + src) + 16 * q);
-    }
+  for (int c = 0; c < kCopies; ++c) {
+    const int row = 4 * (wave * kCopies + c) + (lane >> 4), rr = row & (kRows - 1);
+    src[c] = (row < kRows ? xh : xl) + (size_t)min(m0 + rr, M - 1) * K + 8 * ((lane & 15) ^ (rr & 15));
+  }
+  auto copy_x = [&](int half, int buf) {
+#pragma unroll
+    for (int c = 0; c < kCopies; ++c)
+      copy16_to_lds(src[c] + (size_t)half * 128, uniform(lds0 + buf * kBuf + (wave * kCopies + c) * 1024));
   };
-  auto store_x = [&](uint8_t* buf) {
+
+  f32x16 acc[MTW];
 #pragma unroll
-    for (int i = 0; i < kPieces; ++i) {
-      const int p = tid + 64 * kIq4Waves * i, r = p >> 6, pc = p & 63, part = pc >> 5, q = pc & 31;
-      *(u32x4a4*)(buf + part * kRows * kXStride + r * kXStride + 16 * q) = stage[i];
-    }
-  };
-  IQ4W cur[NT], nxt[NT];
-#pragma unroll
-  for (int nt = 0; nt < NT; ++nt) cur[nt] = load_iq4(row[nt], 0, g);
-  load_x(0);
-  store_x(smem);
+  for (int mt = 0; mt < MTW; ++mt) acc[mt] = kZero16;
+  copy_x(0, 0);
+  pw.copy(0, slot0);
+  wait_vmcnt(0);
   __syncthreads();
   for (int b = 0; b < nb; ++b) {
-    if (b + 1 < nb) {
-      load_x(b + 1);
+    u32x2a4 hdr, qs[8];
+    {
+      const uint8_t* p = smem + slot + pw.at(b, r);
+      hdr = ld8(p);
 #pragma unroll
-      for (int nt = 0; nt < NT; ++nt) nxt[nt] = load_iq4(row[nt], b + 1, g);
+      for (int t = 0; t < 8; ++t) qs[t] = ld8(p + 8 + 16 * t + 8 * h);
     }
-    const uint8_t* Xh = smem + (b & 1) * kBuf;
-    const uint8_t* Xl = Xh + kRows * kXStride;
-    // sub-block t's scale bits and index words move to the front as t advances (no indexing by
-    // t). Two weight tiles unroll the loop by four (fully unrolled they need more than the 256
-    // VGPRs of two waves per SIMD; rolled, the moves cost 5% more time), one tile fully, where
-    // the moves vanish.
-    float dh[NT];
-    uint32_t shs[NT], sls[NT];
+    const float d = half_to_float(hdr.x);
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt) {
-      dh[nt] = half_to_float(cur[nt].hdr[0]);
-      shs[nt] = cur[nt].hdr[0] >> 16, sls[nt] = cur[nt].hdr[1];
-    }
-#pragma unroll(NT == 1 ? 8 : 4)
-    for (int t = 0; t < 8; ++t) {
-      float dl[NT];
-      bf16x8 bk[NT];
-#pragma unroll
-      for (int nt = 0; nt < NT; ++nt) {
-        const int ls = (int)((sls[nt] & 15u) | ((shs[nt] & 3u) << 4));
-        sls[nt] >>= 4, shs[nt] >>= 2;
-        dl[nt] = dh[nt] * (float)(ls - 32);
-        const uint32_t q0 = cur[nt].qs[0], q1 = cur[nt].qs[1];
-#pragma unroll
-        for (int j = 0; j < 14; ++j) cur[nt].qs[j] = cur[nt].qs[j + 2];
-        const uint32_t i0 = (g >= 2 ? q0 >> 4 : q0) & 0x0F0F0F0Fu, i1 = (g >= 2 ? q1 >> 4 : q1) & 0x0F0F0F0Fu;
-        bk[nt] = __builtin_bit_cast(bf16x8, grid_bf16x8(i0, i1));
+    for (int half = 0; half < 2; ++half) {
+      const bool more = half == 0 || b + 1 < nb;
+      if (more) copy_x(2 * b + half + 1, half ^ 1);
+      if (half == 0 && b + 1 < nb) {
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the weights are in registers
+        __builtin_amdgcn_sched_barrier(0);
+        pw.copy(b + 1, slot0);
       }
+      const uint8_t* X = smem + half * kBuf;
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt) {
-        const int off = (16 * mt + ln) * kXStride + 2 * (32 * t + 8 * g);
-        const bf16x8 ah = __builtin_bit_cast(bf16x8, *(const u32x4*)(Xh + off));
-        const bf16x8 al = __builtin_bit_cast(bf16x8, *(const u32x4*)(Xl + off));
+      for (int tt = 0; tt < 4; ++tt) {
+        const int t = 4 * half + tt;
+        const int ls = (int)(((hdr.y >> (4 * t)) & 15u) | (((hdr.x >> (16 + 2 * t)) & 3u) << 4));
+        const float dl = d * (float)(ls - 32);
+        const uint32_t q0 = qs[t].x, q1 = qs[t].y;
+        const bf16x8 b0 = __builtin_bit_cast(bf16x8, grid_bf16x8(q0 & 0x0F0F0F0Fu, q1 & 0x0F0F0F0Fu));
+        const bf16x8 b1 = __builtin_bit_cast(bf16x8, grid_bf16x8((q0 >> 4) & 0x0F0F0F0Fu, (q1 >> 4) & 0x0F0F0F0Fu));
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt) {
-          f32x4 D = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, bk[nt], f32x4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
-          D = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, bk[nt], D, 0, 0, 0);
+        for (int mt = 0; mt < MTW; ++mt) {
+          const uint8_t* xr = X + (32 * mt + r) * 256;
+          auto a = [&](int part, int step) {
+            return __builtin_bit_cast(bf16x8, *(const u32x4*)(xr + part * kRows * 256 +
+                                                              16 * ((4 * tt + 2 * step + h) ^ (r & 15))));
+          };
+          f32x16 D = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a(0, 0), b0, kZero16, 0, 0, 0);
+          D = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a(0, 1), b1, D, 0, 0, 0);
+          D = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a(1, 0), b0, D, 0, 0, 0);
+          D = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a(1, 1), b1, D, 0, 0, 0);
 #pragma unroll
-          for (int i = 0; i < 4; ++i) acc[mt][nt][i] = fmaf(dl[nt], D[i], acc[mt][nt][i]);
+          for (int i = 0; i < 16; ++i) acc[mt][i] = fmaf(dl, D[i], acc[mt][i]);
         }
       }
-      __builtin_amdgcn_sched_barrier(0);  // one sub-block's operands live at a time
-    }
-    if (b + 1 < nb) {
-      store_x(smem + ((b + 1) & 1) * kBuf);
 #pragma unroll
-      for (int nt = 0; nt < NT; ++nt) cur[nt] = nxt[nt];
+      for (int mt = 0; mt < MTW; ++mt) asm volatile("" : "+v"(acc[mt]));
+      wait_vmcnt(0);    // this wave's pieces of the next half block are in LDS
+      __syncthreads();  // everyone's are, and everyone is done with this one
     }
-    __syncthreads();
   }
+  if (n < N) {
 #pragma unroll
-  for (int nt = 0; nt < NT; ++nt) {
-    const int n = n0 + 16 * nt + ln;
+    for (int mt = 0; mt < MTW; ++mt)
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int m = m0 + 16 * mt + 4 * g + i;
-        if (m < M && n < N) y.put((size_t)m * ldy + n, acc[mt][nt][i]);
+      for (int i = 0; i < 16; ++i) {
+        const int m = m0 + 32 * mt + 8 * (i >> 2) + 4 * h + (i & 3);
+        if (m < M) y.put((size_t)m * ldy + n, acc[mt][i]);
       }
   }
 }
@@ -219,23 +185,23 @@ int launch_iq4_prefill(const uint8_t* w, long long row_bytes, const float* x, vo
   const long long n4 = (long long)m_rows * k / 4;
   hipLaunchKernelGGL(split_bf16_kernel, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, stream, x, hi,
                      lo, n4);
-  constexpr int MT = 4;
-  constexpr int kLds = 2 * 2 * 16 * MT * kXStride;
-  const int mblocks = (m_rows + 16 * MT - 1) / (16 * MT);
-  auto go = [&](auto kern, int wg_rows) {
-    allow_lds((const void*)kern, kLds);
-    const dim3 grid((n_rows + wg_rows - 1) / wg_rows, mblocks);
-    hipLaunchKernelGGL(kern, grid, dim3(64 * kIq4Waves), kLds, stream, w, row_bytes, hi, lo, k, y,
-                       ldy, m_rows, n_rows);
+  const int pieces = ppieces<PIQ4>(((uintptr_t)w & 7) == 0);
+  auto go = [&](auto kern, int wn, int mtw) {
+    const int lds = 2 * 2 * 32 * mtw * 256 + wn * pslot_bytes(pieces);
+    allow_lds((const void*)kern, lds);
+    const dim3 grid((n_rows + 32 * wn - 1) / (32 * wn), (m_rows + 32 * mtw - 1) / (32 * mtw));
+    hipLaunchKernelGGL(kern, grid, dim3(64 * wn), lds, stream, w, row_bytes, hi, lo, k, y, ldy, m_rows,
+                       n_rows, pieces);
     return 0;
   };
-  // two weight tiles per wave where that still gives at least two rounds of workgroups (measured
-  // on MI355X per call, the same bits: 4096 x 4096 M = 2048 302 vs 340-347 us, 14336 x 4096
-  // M = 2048 947 vs 1105; at M = 512 the halved grid left CUs idle, 153 vs 96 us)
-  constexpr int kRows2 = 16 * 2 * kIq4Waves;
-  if ((long long)((n_rows + kRows2 - 1) / kRows2) * mblocks >= 2LL * cu_count())
-    return go(iq4_mtile_kernel<MT, 2>, kRows2);
-  return go(iq4_mtile_kernel<MT, 1>, 16 * kIq4Waves);
+  // Two activation tiles share a wave's looked-up weights, and eight waves an activation block in LDS,
+  // while the grid fills the chip. Measured on MI355X, us per call with the split, eight waves of two
+  // tiles / four of two / two of one: 4096 x 4096 M = 2048 (512 workgroups of the first form) 200 / 215 /
+  // 326, M = 512 (128) 86 / 58 / 93, M = 64 (16) 79 / 52 / 40; 14336 x 4096 M = 512 (448) 169 / 203 / 273.
+  const long long m_tiles = (m_rows + 63) / 64, cus = cu_count();
+  if ((n_rows + 255) / 256 * m_tiles >= cus) return go(iq4_ptile_kernel<8, 2>, 8, 2);
+  if ((n_rows + 127) / 128 * m_tiles >= cus * 3 / 4) return go(iq4_ptile_kernel<4, 2>, 4, 2);
+  return go(iq4_ptile_kernel<2, 1>, 2, 1);
 }
 
 }  // namespace mxa

@@ -29,6 +29,7 @@
 // Numerics: integer sums are exact and the fp32 steps are the oracle's, in block order, so the
 // outputs equal the decode kernels' bit for bit.
 #include "mxa_kernels.hpp"
+#include "mxa_pcopy.hpp"
 #include "mxa_tiles.hpp"
 
 #pragma clang fp contract(off)
@@ -128,8 +129,7 @@ struct PQ4 {
   struct W {
     u32x4a4 hdr, q[4];
   };
-  static constexpr int kBytes = 144;
-  static constexpr bool kShifts = false;
+  static constexpr int kBytes = 144, kShift = 0;
   __device__ __forceinline__ static W load(const uint8_t* lds, int off, int h) {
     const uint8_t* p = lds + off;
     W w;
@@ -190,8 +190,7 @@ struct PQ6 {
     u32x4a4 ql[4], qh[2], sc;  // ql[64 hh + 32 q + 16 h ..] at 2 hh + q, qh[32 hh + 16 h ..]
     uint32_t d;
   };
-  static constexpr int kBytes = 210;
-  static constexpr bool kShifts = true;
+  static constexpr int kBytes = 210, kShift = 14;
   // 16 bytes from a 2-byte aligned place, by dwords and v_alignbyte (sh = 0 takes no byte of e)
   __device__ __forceinline__ static u32x4a4 ld16_a2(const uint8_t* base, uint32_t sh) {
     const u32x4a4 v = ld16(base);
@@ -266,8 +265,7 @@ struct PQ8 {
     u32x4a4 e[4], o[4];
     uint32_t x[4];  // dword 4 h + 4: the end of the even quants (h = 1: and the odd block's d)
   };
-  static constexpr int kBytes = 272;
-  static constexpr bool kShifts = false;
+  static constexpr int kBytes = 272, kShift = 0;
   __device__ __forceinline__ static W load(const uint8_t* lds, int off, int h) {
     const uint8_t* p = lds + off + 16 * h;
     W w;
@@ -323,58 +321,6 @@ template <> struct PTileOf<T_Q8_0> { using T = PQ8; };
 
 // LDS bytes of one block of `rows` activation rows: q8 | bsums (fp16) | d.
 constexpr int pbuf_bytes(int rows) { return rows * (QK + 32 + 4); }
-// 16-byte pieces that cover one block of a weight row wherever it starts in its first piece, and a
-// wave's LDS bytes for the 32 rows it owns (whole copies of 64 pieces).
-template <class T>
-__host__ __device__ constexpr int ppieces(bool aligned) {
-  return (T::kBytes + (T::kShifts ? 14 : aligned ? 0 : 12) + 15) / 16;
-}
-constexpr int pslot_bytes(int pieces) { return (32 * pieces + 63) / 64 * 1024; }
-
-__device__ __forceinline__ uint32_t uniform(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
-
-// 4 bytes per lane from `g` to LDS byte address lds + 4 * lane.
-__device__ __forceinline__ void copy4_to_lds(const void* g, uint32_t lds) {
-  asm volatile("global_load_lds_dword %0, off" ::"v"(g), "{m0}"(lds) : "memory");
-}
-
-// A wave's 32 weight rows, copied block by block into a slot that only it reads. Piece c of row q comes
-// from the 16-byte boundary at or below the block's start, so every piece holds at least one byte of the
-// block and none lies outside the 16-byte units that the matrix occupies. Rows >= N repeat row N - 1.
-template <class T>
-struct PWeights {
-  static constexpr int kMax = (32 * ppieces<T>(false) + 63) / 64;
-  const uint8_t* row0;  // the 16-byte boundary at or below the first row
-  uint32_t off[kMax], pc[kMax];
-  uint32_t mine;  // of lane % 32's row from row0
-  int pieces, copies;
-  __device__ __forceinline__ PWeights(const uint8_t* w, long long row_bytes, int n0, int N, int pieces_, int lane)
-      : pieces(pieces_), copies(pslot_bytes(pieces_) >> 10) {
-    const uint32_t mis = (uint32_t)((uintptr_t)w & 15);
-    const long long first = (long long)min(n0, N - 1) * row_bytes;
-    row0 = (const uint8_t*)((uintptr_t)w & ~(uintptr_t)15) + (first & ~15LL);
-    auto row_off = [&](int q) {
-      return mis + (uint32_t)(first & 15) + (uint32_t)((min(n0 + q, N - 1) - min(n0, N - 1)) * row_bytes);
-    };
-#pragma unroll
-    for (int i = 0; i < kMax; ++i) {
-      const int s = min(64 * i + lane, 32 * pieces - 1), q = s / pieces;
-      pc[i] = 16 * (uint32_t)(s - q * pieces);
-      off[i] = row_off(q);
-    }
-    mine = row_off(lane & 31);
-  }
-  __device__ __forceinline__ void copy(int b, uint32_t slot) const {
-#pragma unroll
-    for (int i = 0; i < kMax; ++i)
-      if (i < copies)
-        copy16_to_lds_s(row0, ((off[i] + (uint32_t)(T::kBytes * b)) & ~15u) + pc[i], uniform(slot + 1024 * i));
-  }
-  // where in the slot row r's block b starts
-  __device__ __forceinline__ int at(int b, int r) const {
-    return r * pieces * 16 + (int)((mine + (uint32_t)(T::kBytes * b)) & 15u);
-  }
-};
 
 // The outputs of activation rows m0 .. m0 + 32 MTW - 1 of M.
 template <int TYPE, int WN, int MTW>

@@ -1,4 +1,4 @@
-"""The prefill tiles (mxa_ptile.hip) at the places where they can go wrong, against the oracle bit for
+"""The prefill tiles (mxa_ptile.hip, mxa_iq4.hip) at the places where they can go wrong, against the oracle bit for
 bit: remainders of the 32-row tiles on both sides, one block per row, rows whose blocks start at
 2-byte boundaries, weights that start 4 bytes past a 16-byte boundary, each choice of workgroup, and
 the largest integer sums of each type."""
@@ -9,7 +9,7 @@ import torch
 
 from matricxon_amd import synthetic as S
 from oracle import dequant as D
-from tests.test_gpu_kernels import bits, dev, host
+from tests.test_gpu_kernels import assert_within_tolerance, bits, dev, host
 
 pytestmark = pytest.mark.gpu
 
@@ -83,6 +83,52 @@ def test_grouped_prefill_tiles_match_oracle(gpu, oracle, t, counts) -> None:
     x = S.activations(sum(counts), k, seed=71)
     off = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
     got = host(gpu.matmul_moe(t, dev(w), dev(x), dev(off), max(counts), n, k))
+    for i, c in enumerate(counts):
+        if c:
+            rows = slice(off[i], off[i + 1])
+            assert np.array_equal(bits(got[rows]), bits(oracle.gemm(t, w[i], x[rows], n, k)))
+
+
+@pytest.mark.parametrize("n,k,m,shift", [
+    (1, 256, 17, 0), (33, 512, 33, 0), (70, 768, 64, 4), (70, 1280, 70, 8), (129, 768, 96, 12),
+    (8200, 256, 400, 0),  # four waves, two tiles
+    (16500, 512, 300, 0),  # eight waves, two tiles
+])
+def test_iq4_prefill_tiles_match_oracle(gpu, oracle, n, k, m, shift) -> None:
+    """IQ4_XS on the bf16 tiles: rows whose blocks start at 8-byte multiples, weights at every dword
+    of a 16-byte unit, remainders on both sides; within the type's tolerance."""
+    w = S.packed_weight(D.IQ4_XS, n, k, seed=n + k)
+    x = S.activations(m, k, seed=m)
+    buf = torch.zeros(w.size + 64, dtype=torch.uint8, device="cuda")
+    wd = buf[shift:shift + w.size].view(n, -1)
+    wd.copy_(dev(w))
+    got = host(gpu.matmul(D.IQ4_XS, wd, dev(x), n, k))
+    rows = np.unique(np.concatenate([np.arange(min(n, 200)), np.arange(max(0, n - 200), n)]))
+    assert_within_tolerance(got[:, rows], oracle.gemm(D.IQ4_XS, w[rows], x, len(rows), k))
+
+
+@pytest.mark.parametrize("t", TYPES)
+def test_grouped_prefill_expert_strides(gpu, oracle, t) -> None:
+    """Experts 4 bytes further apart than their rows take: their blocks start at every dword of a 16-byte
+    unit, the last expert's at the end of the allocation."""
+    n, k, e = 300, 512, 5
+    rb = gpu.row_bytes(t, k)
+    stride = -(-n * rb // 16) * 16 + 4
+    w = np.stack([S.packed_weight(t, n, k, seed=80 + i) for i in range(e)])
+    flat = np.zeros((e - 1) * stride + n * rb, dtype=np.uint8)
+    for i in range(e):
+        flat[i * stride:i * stride + n * rb] = w[i].reshape(-1)
+    counts = [33, 40, 1, 0, 64]
+    off = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    x = S.activations(sum(counts), k, seed=81)
+    wd, xd, od = dev(flat), dev(x), dev(off)
+    ws = torch.empty(gpu.workspace_bytes(t, sum(counts), k), dtype=torch.uint8, device="cuda")
+    y = torch.empty((sum(counts), n), dtype=torch.float32, device="cuda")
+    st = gpu._lib.mxa_gemm_moe(t, wd.data_ptr(), stride, e, xd.data_ptr(), od.data_ptr(), sum(counts), 64,
+                               y.data_ptr(), n, k, ws.data_ptr(), ws.numel(),
+                               torch.cuda.current_stream().cuda_stream)
+    assert st == 0
+    got = host(y)
     for i, c in enumerate(counts):
         if c:
             rows = slice(off[i], off[i + 1])
