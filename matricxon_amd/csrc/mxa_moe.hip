@@ -50,85 +50,98 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(
 // p = t * top_k + k has expert e = ids[p] clamped into [0, n_experts); its place in the sorted
 // order is the pairs of smaller experts plus the earlier pairs of the same expert, which is where
 // a stable argsort of the flattened ids puts it (the order the reference's per-expert loop visits
-// tokens: moe_experts.py:81-88, tokens ascending within an expert). Histogram (LDS atomics),
-// exclusive scan over experts, then chunks of 1024 pairs in order: each wave ranks its lanes
-// among equal experts with ballots, the waves' counts are prefixed per expert, and a per-expert
-// base carries from chunk to chunk.
+// tokens: moe_experts.py:81-88, tokens ascending within an expert). Every wave owns a contiguous run of
+// pairs and its own counters, 64 pairs a step: the lanes of one expert find each other with a ballot
+// per bit of the expert id, and the first of them updates the counter. One pass counts; the counts are
+// prefixed over waves and experts; a second pass places.
+//
+// Bound: latency, of a step's ballots and counter and of the ids' loads (four steps requested at a time);
+// the runs need no barrier. A ballot per distinct expert and chunks of 1024 pairs between barriers took
+// 26.5 us at 4096 pairs of 64 experts (kernel alone, MI355X).
 constexpr int kRouteWaves = 16;
 __global__ __launch_bounds__(64 * kRouteWaves) void moe_route_kernel(
     const void* __restrict__ ids, int ids64, int n_pairs, int top_k, int n_experts,
     int32_t* __restrict__ offsets, int32_t* __restrict__ pair_tok, int32_t* __restrict__ rows,
     int32_t* __restrict__ ids32) {
-  __shared__ int cnt[kMoeRouteMaxExperts];
-  __shared__ int scan[2][kMoeRouteMaxExperts];
-  __shared__ int base[kMoeRouteMaxExperts];
-  __shared__ int wcnt[kRouteWaves][kMoeRouteMaxExperts];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  auto raw = [&](int p) -> long long {
-    return ids64 ? ((const long long*)ids)[p] : (long long)((const int32_t*)ids)[p];
-  };
-  auto expert = [&](long long v) { return v < 0 ? 0 : v >= n_experts ? n_experts - 1 : (int)v; };
-  if (tid < kMoeRouteMaxExperts) cnt[tid] = 0;
-  __syncthreads();
-  for (int p = tid; p < n_pairs; p += 64 * kRouteWaves) {
-    const long long v = raw(p);
-    atomicAdd(&cnt[expert(v)], 1);
-    if (ids32 != nullptr) ids32[p] = (int32_t)v;  // torch's int64 -> int32 conversion
-  }
-  __syncthreads();
-  // inclusive scan of the counts (Hillis-Steele over kMoeRouteMaxExperts entries)
-  int cur = 0;
-  if (tid < kMoeRouteMaxExperts) scan[0][tid] = tid < n_experts ? cnt[tid] : 0;
-  for (int off = 1; off < kMoeRouteMaxExperts; off <<= 1) {
-    __syncthreads();
-    if (tid < kMoeRouteMaxExperts) {
-      int x = scan[cur][tid];
-      if (tid >= off) x += scan[cur][tid - off];
-      scan[cur ^ 1][tid] = x;
+  __shared__ int cnt[kRouteWaves][kMoeRouteMaxExperts];
+  __shared__ int part[kMoeRouteMaxExperts / 64];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int bits = n_experts > 1 ? 32 - __builtin_clz(n_experts - 1) : 0;
+  const int run = (n_pairs + 64 * kRouteWaves - 1) / (64 * kRouteWaves) * 64;
+  const int begin = wave * run, end = min(begin + run, n_pairs);
+  const uint64_t below = (1ull << lane) - 1ull;
+  // step(p, valid, v, e, m) for every 64 pairs of the run: m, the lanes of this lane's expert
+  auto walk = [&](auto&& step) {
+    for (int c0 = begin; c0 < end; c0 += 256) {
+      long long v[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int p = min(c0 + 64 * j + lane, n_pairs - 1);
+        v[j] = ids64 ? ((const long long*)ids)[p] : (long long)((const int32_t*)ids)[p];
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        if (c0 + 64 * j >= end) break;
+        const int p = c0 + 64 * j + lane;
+        const bool valid = p < end;
+        const int e = v[j] < 0 ? 0 : v[j] >= n_experts ? n_experts - 1 : (int)v[j];
+        uint64_t m = __ballot(valid);
+        for (int b = 0; b < bits; ++b) {
+          const bool one = (e >> b) & 1;
+          const uint64_t ones = __ballot(one);
+          m &= one ? ones : ~ones;
+        }
+        step(p, valid, v[j], e, m);
+        __builtin_amdgcn_wave_barrier();  // the next step reads the counters that this one wrote
+      }
     }
-    cur ^= 1;
+  };
+#pragma unroll
+  for (int i = 0; i < kMoeRouteMaxExperts / 64; ++i) cnt[wave][64 * i + lane] = 0;
+  __builtin_amdgcn_wave_barrier();
+  walk([&](int p, bool valid, long long v, int e, uint64_t m) {
+    if (!valid) return;
+    if ((m & below) == 0) cnt[wave][e] += __popcll(m);
+    if (ids32 != nullptr) ids32[p] = (int32_t)v;  // torch's int64 -> int32 conversion
+  });
+  __syncthreads();
+  // thread e: the waves' counts of expert e, prefixed; the experts' totals scanned over a wave, then waves
+  int before[kRouteWaves], total = 0, incl = 0;
+  if (tid < kMoeRouteMaxExperts) {
+#pragma unroll
+    for (int w = 0; w < kRouteWaves; ++w) before[w] = cnt[w][tid];
+#pragma unroll
+    for (int w = 0; w < kRouteWaves; ++w) {
+      const int c = before[w];
+      before[w] = total;
+      total += c;
+    }
+    incl = total;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int x = __shfl_up(incl, off, 64);
+      if (lane >= off) incl += x;
+    }
+    if (lane == 63) part[wave] = incl;
   }
   __syncthreads();
-  if (tid < n_experts) {
-    base[tid] = scan[cur][tid] - cnt[tid];
-    offsets[tid] = base[tid];
+  if (tid < kMoeRouteMaxExperts) {
+    int base = incl - total;
+    for (int w = 0; w < wave; ++w) base += part[w];
+    if (tid < n_experts) offsets[tid] = base;
+#pragma unroll
+    for (int w = 0; w < kRouteWaves; ++w) cnt[w][tid] = before[w] + base;
   }
   if (tid == 0) offsets[n_experts] = n_pairs;
-  for (int c0 = 0; c0 < n_pairs; c0 += 64 * kRouteWaves) {
-    for (int i = tid; i < kRouteWaves * kMoeRouteMaxExperts; i += 64 * kRouteWaves)
-      wcnt[i / kMoeRouteMaxExperts][i % kMoeRouteMaxExperts] = 0;
-    __syncthreads();  // also: base is set (first chunk) or carried (later chunks)
-    const int p = c0 + tid;
-    const bool valid = p < n_pairs;
-    const int e = valid ? expert(raw(p)) : -1;
-    int rank = 0;  // earlier lanes of this wave with the same expert
-    uint64_t rem = __ballot(valid);
-    while (rem != 0) {  // wave-uniform: one pass per distinct expert of the wave
-      const int leader = __builtin_ctzll(rem);
-      const int v = __builtin_amdgcn_readlane(e, leader);
-      const uint64_t m = __ballot(valid && e == v);
-      if (valid && e == v) rank = __popcll(m & ((1ull << lane) - 1ull));
-      if (lane == 0) wcnt[wave][v] = __popcll(m);
-      rem &= ~m;
-    }
-    __syncthreads();
-    if (tid < n_experts) {  // the waves' counts prefixed per expert, from the carried base
-      int run = base[tid];
-      for (int w = 0; w < kRouteWaves; ++w) {
-        const int t = wcnt[w][tid];
-        wcnt[w][tid] = run;
-        run += t;
-      }
-      base[tid] = run;
-    }
-    __syncthreads();
-    if (valid) {
-      const int sidx = wcnt[wave][e] + rank;
-      rows[p] = sidx;
-      pair_tok[sidx] = p / top_k;
-    }
-    __syncthreads();  // every lane has read wcnt before the next chunk clears it
-  }
+  __syncthreads();
+  walk([&](int p, bool valid, long long, int e, uint64_t m) {
+    if (!valid) return;
+    const int first = cnt[wave][e], place = first + __popcll(m & below);
+    rows[p] = place;
+    pair_tok[place] = p / top_k;
+    __builtin_amdgcn_wave_barrier();
+    if ((m & below) == 0) cnt[wave][e] = first + __popcll(m);
+  });
 }
 
 }  // namespace

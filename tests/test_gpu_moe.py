@@ -184,7 +184,10 @@ def test_grouped_rows_past_the_bound(gpu, oracle, case) -> None:
 # (n_tokens, top_k, n_experts, id dtype): decode and batched routings, more than one chunk of 1024
 # pairs, more distinct experts than a wave has lanes, ids outside the range, int32 ids
 ROUTE_CASES = [(1, 2, 8, torch.int64), (16, 8, 40, torch.int64), (300, 6, 256, torch.int64),
-               (2000, 4, 64, torch.int32), (5, 3, 1, torch.int64), (1030, 1, 7, torch.int32)]
+               (2000, 4, 64, torch.int32), (5, 3, 1, torch.int64), (1030, 1, 7, torch.int32),
+               # one pair; a wave's run of whole steps; a last wave of one pair; runs of many steps
+               (1, 1, 2, torch.int64), (512, 8, 64, torch.int64), (961, 1, 129, torch.int32),
+               (9001, 4, 9, torch.int64)]
 
 
 @pytest.mark.parametrize("case", range(len(ROUTE_CASES)))
