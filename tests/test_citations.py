@@ -79,7 +79,7 @@ def _citations():
                 yield rel, lineno, m.group(1), m.group(2)
 
 
-@pytest.mark.skipif(not REFERENCE.is_dir(), reason="the reference tree is not present")
+@pytest.mark.skipif(not any(REFERENCE.glob("*")), reason="the reference tree is not present")
 def test_every_citation_points_at_existing_lines():
     bad = []
     for rel, lineno, name, spec in _citations():
