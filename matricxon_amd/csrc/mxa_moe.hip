@@ -56,8 +56,8 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(
 // prefixed over waves and experts; a second pass places.
 //
 // Bound: latency, of a step's ballots and counter and of the ids' loads (four steps requested at a time);
-// the runs need no barrier. A ballot per distinct expert and chunks of 1024 pairs between barriers took
-// 26.5 us at 4096 pairs of 64 experts (kernel alone, MI355X).
+// the runs need no barrier. Measured on MI355X, kernel alone, 4096 pairs of 64 experts: 7.8 us; a ballot
+// per distinct expert of a wave, in chunks of 1024 pairs between barriers, took 26.5.
 constexpr int kRouteWaves = 16;
 __global__ __launch_bounds__(64 * kRouteWaves) void moe_route_kernel(
     const void* __restrict__ ids, int ids64, int n_pairs, int top_k, int n_experts,
