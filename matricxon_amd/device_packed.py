@@ -158,6 +158,9 @@ class DevicePackedLinear(nn.Module):
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         lead = x.shape[:-1]
         k = self.in_features
+        # As F.linear: the rows are passed by address below, so nothing after this compares widths.
+        if x.shape[-1:] != (k,) and x.numel() > 0:
+            raise RuntimeError(f"x must have {k} values in its last dimension, got shape {tuple(x.shape)}")
         if self.backend == "numba":
             return self.finish(self._forward_f32(x.reshape(-1, k)), lead)
         # The reference casts x to the layer dtype before its matmul (device_packed.py:54).
@@ -172,7 +175,7 @@ class DevicePackedLinear(nn.Module):
             y = torch.empty((n, big_n), dtype=torch.bfloat16 if bf16 else torch.float32, device=dev)
             self._gemm.matmul_q8k(self._ggml_type, packed, ws, None, y, n, big_n, k)
         elif bf16 and x.device == dev and n > 0:
-            xb = x if x.dim() == 2 else x.reshape(n, k)
+            xb = x if x.dim() == 2 else x.reshape(n, k)  # of width k: checked above
             if not xb.is_contiguous() or xb.data_ptr() % 16 != 0:
                 xb = xb.clone(memory_format=torch.contiguous_format)
             y = torch.empty((n, big_n), dtype=torch.bfloat16, device=dev)
@@ -201,7 +204,7 @@ class DevicePackedLinear(nn.Module):
         in its dtype, plus bias."""
         if y.dtype != self._dtype:
             y = y.to(self._dtype)
-        if len(lead) != 1:
+        if len(lead) != 1 or lead[0] != y.shape[0]:
             y = y.reshape(*lead, self.out_features)
         return y if self.bias is None else y + self.bias
 
