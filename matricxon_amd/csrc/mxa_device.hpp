@@ -230,6 +230,15 @@ __device__ __forceinline__ void copy16_to_lds_s_nt(const void* base, uint32_t of
   asm volatile("global_load_lds_dwordx4 %0, %1 nt" ::"v"(off), "s"(base), "{m0}"(lds_addr) : "memory");
 }
 
+// Between LDS accesses of different lanes of one wave: what a lane wrote before it, every lane of the wave
+// reads after it. A wave's LDS accesses execute in order, so it costs no instruction; the fence keeps the
+// compiler to that order (the barrier alone only stops its scheduler).
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Grid-order tile index for workgroup `wg` of `n_wg` such that consecutive tiles land on the same
 // XCD: workgroups are dealt to the 8 XCDs round-robin, so XCD x gets a contiguous tile range.
 __device__ __forceinline__ int xcd_tile(int wg, int n_wg) {

@@ -92,13 +92,13 @@ __global__ __launch_bounds__(64 * kRouteWaves) void moe_route_kernel(
           m &= one ? ones : ~ones;
         }
         step(p, valid, v[j], e, m);
-        __builtin_amdgcn_wave_barrier();  // the next step reads the counters that this one wrote
+        wave_sync();  // the next step reads the counters that this one wrote
       }
     }
   };
 #pragma unroll
   for (int i = 0; i < kMoeRouteMaxExperts / 64; ++i) cnt[wave][64 * i + lane] = 0;
-  __builtin_amdgcn_wave_barrier();
+  wave_sync();
   walk([&](int p, bool valid, long long v, int e, uint64_t m) {
     if (!valid) return;
     if ((m & below) == 0) cnt[wave][e] += __popcll(m);
@@ -135,12 +135,13 @@ __global__ __launch_bounds__(64 * kRouteWaves) void moe_route_kernel(
   if (tid == 0) offsets[n_experts] = n_pairs;
   __syncthreads();
   walk([&](int p, bool valid, long long, int e, uint64_t m) {
-    if (!valid) return;
     const int first = cnt[wave][e], place = first + __popcll(m & below);
-    rows[p] = place;
-    pair_tok[place] = p / top_k;
-    __builtin_amdgcn_wave_barrier();
-    if ((m & below) == 0) cnt[wave][e] = first + __popcll(m);
+    if (valid) {
+      rows[p] = place;
+      pair_tok[place] = p / top_k;
+    }
+    wave_sync();  // every lane has read its counter
+    if (valid && (m & below) == 0) cnt[wave][e] = first + __popcll(m);
   });
 }
 
