@@ -2,6 +2,8 @@
 // decode for shapes that the streaming kernels do not take, its grouped MoE form, and the choice of kernel
 // for up to 16 activation rows (more: mxa_ptile.hip). The blocks are folded in order 0..nb-1, so the outputs
 // equal the oracle and the decode kernels bit for bit.
+#include <math.h>
+
 #include "mxa_kernels.hpp"
 #include "mxa_tiles.hpp"
 
@@ -192,6 +194,68 @@ int launch_mt_type(const uint8_t* w, long long row_bytes, const Act& act, YOut y
   return launch_ptile(TYPE, w, row_bytes, act, y, ldy, M, N, stream);
 }
 
+// Tile groups per workgroup of moe_dec_kernel (each group's chunk of activations staged once for all of
+// them): the most of 4, 2, 1 that still gives two workgroups per CU (Q8_0 at most 2: four spill).
+// Measured on MI355X, eager forward of 8 experts top 2 (4096 x 14336; Q4_K gate / up, Q6_K down), the same
+// bits: 16 tokens 498 vs 523 us, 128 tokens 1146 vs 1364; with four groups forced, 40 small experts at 16
+// tokens lost (214 vs 204 us) to the smaller grid.
+int moe_dec_groups(int type, int tiles, int n_experts, int chunks) {
+  for (int gs = type == T_Q8_0 ? 2 : 4; gs > 1; gs >>= 1)
+    if ((long long)((tiles + gs - 1) / gs) * n_experts * chunks >= 2LL * cu_count()) return gs;
+  return 1;
+}
+int moe_dec_tiles(int type, int n_rows) { return type == T_Q6_K ? (n_rows + 15) / 16 : (n_rows + 31) / 32; }
+
+// Estimated times in us of the three forms of a grouped projection with a few rows an expert, kernel alone,
+// weights from HBM:
+// - body: the batched-decode bodies (16-row chunks). Every CU has its share of the weight rows that can be in
+//   use, and walks it 16 rows at a time, parts of 8 blocks of long rows one after another; and there are the
+//   workgroups of experts without rows;
+// - ptile: the prefill tiles (32-row chunks). A workgroup of 128 weight rows walks the blocks;
+// - tile: the decode tile below, 8 blocks a step.
+// A start, the steps that a workgroup takes in a row, and for the last two what the other workgroups of its CU
+// cost. The constants are fitted on MI355X to 2800 calls of two tokens or more (512 to 14336 rows, 2 to 56
+// blocks, 4 to 128 experts, random routings of up to 20 rows an expert); half of the estimates are within 6%,
+// the choice that they give is within 0.5% of the best of the three on average, where a rule on the number of
+// prefill tiles and of rows an expert lost 4%. Some of it, us, prefill tiles / decode bodies: 8 experts
+// top 2, Q4_K 14336 x 4096, 3 / 4 / 6 tokens 47 / 53, 53 / 62, 62 / 63, 36 / 40 / 48 tokens (9 / 10 / 12 rows
+// an expert: from 9 on some expert has a second chunk of 16) 74 / 67, 73 / 75, 73 / 84; Q6_K 4096 x 14336, 4 /
+// 36 / 48 tokens 139 / 135, 140 / 142, 141 / 230; 16 experts top 4, Q6_K 3072 x 2048, 3 / 4 / 5 / 7 / 40 tokens
+// 27 / 31, 32 / 34, 38 / 34, 39 / 34, 39 / 34; Q8_0 2048 x 3072, 4 / 7 / 40 tokens 29 / 24, 31 / 24, 33 / 25; 64
+// experts top 8, Q4_K 1024 x 2048, 4 / 5 / 16 tokens 16 / 16, 17 / 22, 23 / 32. Prefill tiles / decode tile: Q6_K
+// 2048 x 1024, 64 experts top 8, 2 / 4 / 16 tokens 16 / 25, 23 / 42, 39 / 84; 2048 x 7168, 4 experts, 4 / 16 rows
+// 71 / 33, 71 / 34; Q4_K 512 x 1536, 64 experts, 8 / 16 rows 12.2 / 11.9, 12.7 / 16.9.
+struct MoeTimes {
+  double body, ptile, tile;
+};
+MoeTimes moe_times(int type, int n_rows, int nb, int n_experts, int total_rows, int max_rows) {
+  struct Fit {
+    double b0, b1, b2, b3, b4, p0, p1, p2, p3, t0, t1, t2, t3, t4;
+  };
+  static constexpr Fit kQ4 = {3.77, 1.492, 0.044, 0.92, 0.003, 5.84, 1.169, 0.977, 0.218, 4.84, 2.163, 0.739, -0.14, 0.282};
+  static constexpr Fit kQ6 = {5.31, 1.821, 0.065, 1.04, 0.004, 6.59, 2.219, 1.714, 0.169, 4.61, 3.439, 0.536, -0.36, 0.377};
+  static constexpr Fit kQ8 = {4.02, 0.983, 0.133, 1.04, 0.004, 6.54, 1.744, 1.515, 0.209, 3.61, 7.086, 0.708, -0.21, 0.552};
+  const Fit& f = type == T_Q4_K ? kQ4 : type == T_Q6_K ? kQ6 : kQ8;
+  const double cus = cu_count(), most = min(n_experts, total_rows), rows = (double)total_rows / n_experts;
+  // experts with rows: as many as max_rows tokens name that choose total_rows / max_rows experts each at random
+  const double choices = (double)total_rows / max_rows;
+  const double named = n_experts * (1 - pow(1 - fmin(1, choices / n_experts), max_rows));
+  const double busy = fmin(most, fmax(named, fmax(1, choices)));
+  const double second = fmin(1, fmax(0, (rows - 8.5) / 5));  // some expert's second chunk of 16 rows
+  MoeTimes t;
+  const double share = ceil(n_rows * most / cus);
+  const int parts = nb <= 16 ? 1 : (nb + 7) / 8;
+  t.body = f.b0 + ceil(share / 16) * parts * (f.b1 + f.b2 * min(nb, parts > 1 ? 8 : 16)) * (1 + f.b3 * second) +
+           f.b4 * ceil(n_rows / share) * (n_experts + (total_rows + 15) / 16);
+  const double xp = (n_rows + 127) / 128 * busy / cus;  // workgroups per CU
+  t.ptile = f.p0 + nb * (f.p1 + f.p2 * fmax(0, ceil(xp - 0.02) - 1) + f.p3 * fmin(1, xp));
+  const int tiles = moe_dec_tiles(type, n_rows);
+  const int gs = moe_dec_groups(type, tiles, n_experts, (max_rows + 15) / 16);
+  const double xt = (tiles + gs - 1) / gs * busy * (1 + 0.5 * second) / cus;
+  t.tile = f.t0 + gs * ((nb + 7) / 8 * f.t1 + nb * f.t4) * (1 + f.t2 * fmax(0, ceil(xt - 0.02) - 1) + f.t3 * fmin(1, xt));
+  return t;
+}
+
 }  // namespace
 
 bool mtile_supported(int type) { return type == T_Q4_K || type == T_Q6_K || type == T_Q8_0; }
@@ -204,42 +268,22 @@ int launch_moe_dec(int type, const uint8_t* w, long long row_bytes, long long ex
     return -1;
   const int chunks = (max_rows + 15) / 16;
   if (chunks > 65535) return -1;
-  // The prefill tiles (32- or 64-row chunks, 128 weight rows a workgroup), except
-  // - where the routing gives too few of them to fill the chip, and where the experts of a large matrix
-  //   have two to eight rows on average: the batched-decode bodies (16-row chunks, every CU a share of
-  //   the rows, all of it requested early), if they take the shape;
-  // - few tiles of shapes that those do not take: the decode tile below.
-  // Measured on MI355X, weights from HBM, us, kernel alone, prefill tiles / the other form: 64 experts
-  // top 8, Q4_K 1024 x 2048, 1 token (64 tiles) 13.1 / 8.8, 4 (256) 15.5 / 14.9, 16 (1 row a expert and
-  // more) 22 / 31, Q6_K 2048 x 1024 (decode tile), 2 / 4 / 16 tokens 15 / 27, 22 / 47, 37 / 81; 8 experts
-  // top 2, Q4_K 14336 x 4096, 4 / 16 / 32 / 48 / 96 tokens 52 / 62, 70 / 63, 69 / 63, 73 / 118, 72 / 120,
-  // Q6_K 4096 x 14336, 2 tokens (128 tiles) 134 / 73, 16 138 / 139, 96 138 / 277; 16 experts top 4, Q6_K
-  // 3072 x 2048, 4 / 16 tokens 24 / 33, 38 / 34; 4 experts top 1, Q6_K 14336 x 4096, 8 tokens 67 / 46; 40
-  // experts top 8 (decode tile), Q4_K 512 x 1536, 4 / 16 tokens (128 / 160 tiles) 10.7 / 7.7, 11.0 / 14.7,
-  // Q6_K 1536 x 512, 1 token (96) 8.6 / 15.2.
+  // The form that should take least time while the experts have few rows (20 on average), the prefill tiles
+  // past that.
+  const MoeTimes est = moe_times(type, n_rows, act.nb, n_experts, total_rows, max_rows);
+  const bool decode = total_rows <= 20LL * n_experts;
   constexpr int kMoeDecodeBodyMaxRows = 96, kMoeDecodeBodyMinN = 1024;
-  const long long busy = total_rows < n_experts ? total_rows : n_experts;
-  const long long chunks32 = (total_rows + 31) / 32;
-  const long long tiles = (n_rows + 127) / 128 * (busy > chunks32 ? busy : chunks32);
-  const bool streams = n_rows >= 2048 && total_rows >= 2LL * n_experts && total_rows <= 8LL * n_experts;
-  if ((tiles < cu_count() || streams) && max_rows <= kMoeDecodeBodyMaxRows && n_rows >= kMoeDecodeBodyMinN &&
+  if (decode && est.body <= fmin(est.ptile, est.tile) && max_rows <= kMoeDecodeBodyMaxRows &&
+      n_rows >= kMoeDecodeBodyMinN &&
       launch_moe_bwave(type, w, row_bytes, expert_stride, n_experts, act, offsets, total_rows, y,
                        ldy, n_rows, stream) == 0)
     return 0;
-  if ((max_rows > 32 || tiles >= (type == T_Q6_K ? 64 : 160)) &&
+  if ((!decode || est.ptile <= est.tile) &&
       launch_moe_ptile(type, w, row_bytes, expert_stride, n_experts, act, offsets, total_rows, y, ldy, n_rows,
                        stream) == 0)
     return 0;
-  // Tile groups per workgroup (each group's chunk of activations staged once for all of them):
-  // the most of 4, 2, 1 that still gives two workgroups per CU (Q8_0 at most 2: four spill).
-  // Measured on MI355X, eager forward of 8 experts top 2 (4096 x 14336; Q4_K gate / up, Q6_K
-  // down), the same bits: 16 tokens 498 vs 523 us, 128 tokens 1146 vs 1364; with four groups
-  // forced, 40 small experts at 16 tokens lost (214 vs 204 us) to the smaller grid.
-  auto go = [&](auto k1, auto k2, auto k4, int rt, int gmax) {
-    const long long want = 2LL * cu_count();
-    const int t1 = (n_rows + 16 * rt - 1) / (16 * rt);
-    auto grid_of = [&](int gs) { return (long long)((t1 + gs - 1) / gs) * n_experts * chunks; };
-    const int gs = gmax >= 4 && grid_of(4) >= want ? 4 : gmax >= 2 && grid_of(2) >= want ? 2 : 1;
+  auto go = [&](auto k1, auto k2, auto k4, int rt) {
+    const int t1 = (n_rows + 16 * rt - 1) / (16 * rt), gs = moe_dec_groups(type, t1, n_experts, chunks);
     const dim3 grid((t1 + gs - 1) / gs, n_experts, chunks);
     if (gs == 4)
       hipLaunchKernelGGL(k4, grid, dim3(256), 0, stream, w, row_bytes, expert_stride, act, offsets,
@@ -255,13 +299,13 @@ int launch_moe_dec(int type, const uint8_t* w, long long row_bytes, long long ex
   switch (type) {
     case T_Q4_K:
       return go(moe_dec_kernel<T_Q4_K, 2, 1>, moe_dec_kernel<T_Q4_K, 2, 2>,
-                moe_dec_kernel<T_Q4_K, 2, 4>, 2, 4);
-    case T_Q8_0:  // k4 is never taken (gmax 2): the two-group form stands in
+                moe_dec_kernel<T_Q4_K, 2, 4>, 2);
+    case T_Q8_0:  // k4 is never taken (at most two groups): the two-group form stands in
       return go(moe_dec_kernel<T_Q8_0, 2, 1>, moe_dec_kernel<T_Q8_0, 2, 2>,
-                moe_dec_kernel<T_Q8_0, 2, 2>, 2, 2);
+                moe_dec_kernel<T_Q8_0, 2, 2>, 2);
     case T_Q6_K:
       return go(moe_dec_kernel<T_Q6_K, 1, 1>, moe_dec_kernel<T_Q6_K, 1, 2>,
-                moe_dec_kernel<T_Q6_K, 1, 4>, 1, 4);
+                moe_dec_kernel<T_Q6_K, 1, 4>, 1);
     default: return -1;
   }
 }

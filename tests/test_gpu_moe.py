@@ -76,29 +76,25 @@ def test_grouped_rows_match_oracle(gpu, oracle, ggml_type, n, k, ci) -> None:
     assert_bit_exact(got.cpu().numpy(), want, "Q8_K given")
 
 
-# Expert matrices of 4096 rows and more at bounds up to 32 rows (16-row chunks through the prefill
-# tile body), and mid-sized ones over many experts, for which the decode tile stages each
-# activation chunk once for two or four groups of weight tiles per workgroup (the most that still
-# gives two workgroups per CU; Q8_0 at most two); N past a whole tile, an empty expert, one past
-# 16 rows.
+# Expert matrices of 4096 rows and more at bounds up to 32 rows, and mid-sized ones over many experts; N past
+# a whole tile, an empty expert, one past 16 rows.
 _MANY = [int(c) for c in np.random.default_rng(5).integers(0, 4, 40)]
 GROUPED_LARGE = [(D.Q4_K, 8200, 1024, [3, 0, 5, 16, 1, 17, 2, 4]),
                  (D.Q6_K, 4100, 2048, [3, 0, 5, 16, 1, 17, 2, 4]),
                  (D.Q8_0, 8200, 512, [3, 0, 5, 16, 1, 17, 2, 4]),
                  (D.Q4_K, 4096, 1024, [2, 7, 1, 0, 9, 3, 16, 5]),
                  (D.Q4_K, 4000, 256, _MANY), (D.Q8_0, 3000, 256, _MANY), (D.Q6_K, 3000, 512, _MANY),
-                 # up to 16 rows per expert on the batched-decode body: resident and ring forms
+                 # up to 16 rows per expert
                  (D.Q6_K, 4100, 2048, [3, 0, 5, 16, 1, 12, 2, 4]),
                  (D.Q8_0, 8200, 1024, [16, 1, 0, 7, 9]),
                  (D.Q4_K, 14336, 1024, [2, 7, 1, 0, 9, 3, 16, 5]),
-                 # long rows (more than 16 blocks) on the batched-decode body
+                 # long rows (more than 16 blocks)
                  (D.Q6_K, 4096, 14336, [3, 0, 5, 16, 1, 12, 2, 4]),
                  (D.Q4_K, 4100, 5120, [16, 2, 0, 9]), (D.Q8_0, 4096, 8192, [5, 16, 1]),
-                 # bounds up to 96: several 16-row chunks of one expert; past 96 the prefill
-                 # tile body
+                 # several chunks of one expert
                  (D.Q6_K, 4096, 5120, [64, 0, 33, 1, 17]), (D.Q4_K, 4096, 1024, [48, 50, 3]),
                  (D.Q4_K, 4096, 1024, [90, 5, 70]), (D.Q6_K, 4096, 1024, [100, 3, 0, 40]),
-                 # expert matrices of 1024 to 4096 rows on the batched-decode bodies
+                 # expert matrices of 1024 to 4096 rows
                  (D.Q4_K, 1024, 2048, [5, 0, 9, 16, 2]), (D.Q6_K, 2048, 1024, [3, 17, 1]),
                  (D.Q8_0, 1500, 4096, [7, 0, 2]), (D.Q6_K, 3072, 5120, [2, 11, 0, 4])]
 
@@ -121,7 +117,7 @@ def test_grouped_rows_large_experts_match_oracle(gpu, oracle, case) -> None:
 
 @pytest.mark.parametrize("ggml_type", TYPES)
 def test_grouped_rows_many_per_expert_match_oracle(gpu, oracle, ggml_type) -> None:
-    """Bounds past 32 rows per expert take 64-row chunks through the prefill tile body: experts
+    """More than 32 rows per expert on average take 64-row chunks on the prefill tiles: experts
     with 0, 1, 63 / 64 / 65 and 150 rows (three chunks), N past a whole 128-row tile."""
     counts = [0, 150, 3, 70, 0, 64, 65, 1, 63]
     n, k = 700, 512
@@ -135,6 +131,36 @@ def test_grouped_rows_many_per_expert_match_oracle(gpu, oracle, ggml_type) -> No
         if counts[e]:
             want = oracle.gemm(ggml_type, w[e], x[off[e]:off[e + 1]], n, k)
             assert_bit_exact(got[off[e]:off[e + 1]], want, f"expert {e}")
+
+
+# Every form of the grouped launch and every type, N past a tile, an empty expert, one past 16 rows: the
+# batched-decode bodies (rows of a CU resident, in a ring, long rows), the 32-row prefill tiles (past 20 rows
+# an expert on average) and, past the 256 experts that those list, two or four tile groups per workgroup
+_300 = [int(c) for c in np.random.default_rng(6).integers(0, 3, 299)] + [17]
+FORMS = ([(D.Q4_K, 1040, 2048, [5, 0, 17, 3]), (D.Q6_K, 1030, 4096, [5, 17, 3]),
+          (D.Q8_0, 1040, 2048, [5, 0, 17, 3])] +
+         [(D.Q4_K, 4100, 4096, [5, 0, 17, 3, 1, 8, 2, 4]), (D.Q6_K, 4100, 4096, [5, 0, 17, 3, 1, 8, 2, 4]),
+          (D.Q8_0, 2050, 3072, [5, 0, 17, 3, 1, 2, 0, 1, 1, 1, 2, 0, 3, 1, 1, 4])] +
+         [(t, 1040, 6144, [5, 0, 17]) for t in TYPES] +
+         [(t, 300, 1280, [5, 31, 32, 33, 1, 40]) for t in TYPES] +
+         [(D.Q4_K, 70, 512, _300), (D.Q4_K, 250, 256, _300), (D.Q6_K, 40, 512, _300), (D.Q6_K, 120, 256, _300),
+          (D.Q8_0, 250, 512, _300)])
+
+
+@pytest.mark.parametrize("case", range(len(FORMS)))
+def test_grouped_forms_match_oracle(gpu, oracle, case) -> None:
+    t, n, k, counts = FORMS[case]
+    w = expert_weights(t, len(counts), n, k, seed=300 + case)
+    x = S.activations(sum(counts), k, seed=330 + case)
+    off = offsets_of(counts)
+    bound = 16 if counts is _300 else max(counts)  # the tile's chunks loop over the last expert's 17 rows
+    got = gpu.matmul_moe(t, torch.from_numpy(w).cuda(), torch.from_numpy(x).cuda(),
+                         torch.from_numpy(off).cuda(), bound, n, k).cpu().numpy()
+    rows = np.unique(np.concatenate([np.arange(0, n, 37), np.arange(max(0, n - 40), n)]))
+    for e, c in enumerate(counts):
+        if c:
+            want = oracle.gemm(t, np.ascontiguousarray(w[e][rows]), x[off[e]:off[e + 1]], len(rows), k)
+            assert_bit_exact(got[off[e]:off[e + 1]][:, rows], want, f"expert {e}")
 
 
 def test_grouped_rows_with_loose_bound(gpu, oracle) -> None:
@@ -153,9 +179,8 @@ def test_grouped_rows_with_loose_bound(gpu, oracle) -> None:
                              oracle.gemm(t, w[e], x[off[e]:off[e + 1]], n, k), f"expert {e}")
 
 
-# (type, N, K, bound, counts): the decode tile (its chunks loop), the 64-row prefill body (bound
-# past 32), the 16-row one (N >= 4096) and the batched-decode bodies (N >= 4096, bound <= 16,
-# resident, ring and long-row forms), each with experts past the bound
+# (type, N, K, bound, counts), each with experts past the bound: the decode tile (its chunks loop), the
+# prefill tiles (64-row chunks, 32-row chunks) and the batched-decode bodies
 PAST_BOUND = [(D.Q6_K, 256, 1024, 16, [40, 0, 3, 33]), (D.Q4_K, 300, 512, 40, [130, 0, 3, 81]),
               (D.Q6_K, 4100, 256, 16, [40, 0, 3, 33]), (D.Q8_0, 4100, 256, 20, [70, 1, 0, 45]),
               (D.Q4_K, 4096, 1024, 16, [40, 0, 3, 17]),
@@ -265,8 +290,7 @@ MODULE_CASES = [
     ((D.Q6_K, D.Q6_K, D.Q4_K), 8, 256, 512, 1, 2, torch.float32),
     # one bfloat16 token through the fused steps, the down projection on 56-block rows
     ((D.Q4_K, D.Q4_K, D.Q6_K), 4, 1024, 14336, 1, 2, torch.bfloat16),
-    # batched-decode bodies for the grouped projections (experts of 1024 rows and more, bounds
-    # up to 96): OLMoE-like 64 experts top 8, long down rows, float32 and Q8_0 down
+    # experts of 1024 rows and more: OLMoE-like 64 experts top 8, long down rows, float32 and Q8_0 down
     ((D.Q4_K, D.Q4_K, D.Q6_K), 64, 2048, 1024, 16, 8, torch.bfloat16),
     ((D.Q4_K, D.Q4_K, D.Q6_K), 64, 2048, 1024, 64, 8, torch.bfloat16),
     ((D.Q4_K, D.Q4_K, D.Q6_K), 8, 1024, 5120, 12, 2, torch.bfloat16),
@@ -311,8 +335,7 @@ def test_module_repeated_expert_in_a_tokens_routing(dtype) -> None:
 
 @pytest.mark.parametrize("n_tokens,ffn", [(40, 256), (20, 4096)])
 def test_module_repeated_expert_past_the_bound_on_prefill_tiles(n_tokens, ffn) -> None:
-    """The same repeated routing where the grouped launch takes the prefill tile body: a bound
-    past 32 rows (64-row chunks) and a 4096-row expert matrix (16-row chunks)."""
+    """The same repeated routing at a bound past 32 rows and with a 4096-row expert matrix."""
     types = (D.Q4_K, D.Q4_K, D.Q6_K)
     mod, per_expert = build_experts(types, 4, 512, ffn, torch.bfloat16, seed=34)
     _check_repeated_routing(mod, per_expert, n_tokens, 512)
@@ -335,8 +358,8 @@ def test_module_rejects_types_without_a_kernel() -> None:
         HipPackedMoEExperts(z, z, z, 13, 13, 13, 256, 256, F.silu)
 
 
-# the grouped launch's bodies: the 16-row decode tile (small bounds, 40 experts), the 64-row
-# prefill tile (bounds past 32) and, for IQ4_XS, the float-row kernel
+# the grouped launch's forms: the decode tile, the prefill tiles (64-row chunks, 32-row ones over 40
+# experts) and, for IQ4_XS, the float-row kernel
 GROUPED_BF16 = [(D.Q4_K, 512, 1024, COUNTS[0]), (D.Q6_K, 300, 2048, COUNTS[0]),
                 (D.Q8_0, 700, 512, [0, 150, 3, 70, 0, 64, 65, 1, 63]),
                 (D.Q4_K, 700, 512, [0, 150, 3, 70, 0, 64, 65, 1, 63]),

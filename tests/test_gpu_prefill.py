@@ -74,7 +74,8 @@ def test_prefill_largest_sums(gpu, oracle, t, sign) -> None:
 
 @pytest.mark.parametrize("t", TYPES)
 @pytest.mark.parametrize("counts", [
-    [0, 1, 31, 32, 33, 2],  # 32-row chunks
+    [0, 1, 31, 32, 33, 2],
+    [5, 1, 31, 32, 33, 40],  # 32-row chunks (past 20 rows an expert on average)
     [0, 1, 64, 65, 33, 0, 129],  # 64-row chunks, the last one of some experts with one tile's rows
 ])
 def test_grouped_prefill_tiles_match_oracle(gpu, oracle, t, counts) -> None:
