@@ -185,23 +185,28 @@ int launch_iq4_prefill(const uint8_t* w, long long row_bytes, const float* x, vo
   const long long n4 = (long long)m_rows * k / 4;
   hipLaunchKernelGGL(split_bf16_kernel, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, stream, x, hi,
                      lo, n4);
-  const int pieces = ppieces<PIQ4>(((uintptr_t)w & 7) == 0);
-  auto go = [&](auto kern, int wn, int mtw) {
-    const int lds = 2 * 2 * 32 * mtw * 256 + wn * pslot_bytes(pieces);
-    allow_lds((const void*)kern, lds);
-    const dim3 grid((n_rows + 32 * wn - 1) / (32 * wn), (m_rows + 32 * mtw - 1) / (32 * mtw));
-    hipLaunchKernelGGL(kern, grid, dim3(64 * wn), lds, stream, w, row_bytes, hi, lo, k, y, ldy, m_rows,
-                       n_rows, pieces);
-    return 0;
+  auto launch = [&](const uint8_t* w, YOut y, int n_rows) {
+    const int pieces = ppieces<PIQ4>(((uintptr_t)w & 7) == 0);
+    auto go = [&](auto kern, int wn, int mtw) {
+      const int lds = 2 * 2 * 32 * mtw * 256 + wn * pslot_bytes(pieces);
+      allow_lds((const void*)kern, lds);
+      const dim3 grid((n_rows + 32 * wn - 1) / (32 * wn), (m_rows + 32 * mtw - 1) / (32 * mtw));
+      hipLaunchKernelGGL(kern, grid, dim3(64 * wn), lds, stream, w, row_bytes, hi, lo, k, y, ldy, m_rows,
+                         n_rows, pieces);
+    };
+    // Two activation tiles share a wave's looked-up weights, and eight waves an activation block in LDS,
+    // while the grid fills the chip. Measured on MI355X, us per call with the split, eight waves of two
+    // tiles / four of two / two of one: 4096 x 4096 M = 2048 (512 workgroups of the first form) 200 / 215 /
+    // 326, M = 512 (128) 86 / 58 / 93, M = 64 (16) 79 / 52 / 40; 14336 x 4096 M = 512 (448) 169 / 203 / 273.
+    const long long m_tiles = (m_rows + 63) / 64, cus = cu_count();
+    if ((n_rows + 255) / 256 * m_tiles >= cus) go(iq4_ptile_kernel<8, 2>, 8, 2);
+    else if ((n_rows + 127) / 128 * m_tiles >= cus * 3 / 4) go(iq4_ptile_kernel<4, 2>, 4, 2);
+    else go(iq4_ptile_kernel<2, 1>, 2, 1);
   };
-  // Two activation tiles share a wave's looked-up weights, and eight waves an activation block in LDS,
-  // while the grid fills the chip. Measured on MI355X, us per call with the split, eight waves of two
-  // tiles / four of two / two of one: 4096 x 4096 M = 2048 (512 workgroups of the first form) 200 / 215 /
-  // 326, M = 512 (128) 86 / 58 / 93, M = 64 (16) 79 / 52 / 40; 14336 x 4096 M = 512 (448) 169 / 203 / 273.
-  const long long m_tiles = (m_rows + 63) / 64, cus = cu_count();
-  if ((n_rows + 255) / 256 * m_tiles >= cus) return go(iq4_ptile_kernel<8, 2>, 8, 2);
-  if ((n_rows + 127) / 128 * m_tiles >= cus * 3 / 4) return go(iq4_ptile_kernel<4, 2>, 4, 2);
-  return go(iq4_ptile_kernel<2, 1>, 2, 1);
+  const int step = prow_limit(row_bytes);
+  for (long long n0 = 0; n0 < n_rows; n0 += step)
+    launch(w + n0 * row_bytes, y.at(n0), (int)min((long long)step, n_rows - n0));
+  return 0;
 }
 
 }  // namespace mxa

@@ -22,6 +22,13 @@ __device__ __forceinline__ void copy4_to_lds(const void* g, uint32_t lds) {
   asm volatile("global_load_lds_dword %0, off" ::"v"(g), "{m0}"(lds) : "memory");
 }
 
+// Weight rows that one launch takes: a lane's offset from its wave's first row has 32 bits, which 32 rows of
+// 128 MiB (K past 10^8) outgrow.
+inline int prow_limit(long long row_bytes) {
+  const long long rows = ((1LL << 32) - 512) / row_bytes;
+  return rows >= 32 ? 0x7FFFFFFF : rows > 1 ? (int)rows : 1;
+}
+
 // A wave's 32 weight rows, copied block by block into a slot that only it reads. Piece c of row q comes
 // from the 16-byte boundary at or below the block's start. Every piece holds at least one byte of the
 // block (`clamp`: a piece that could lie past a block that starts at the boundary repeats the last one

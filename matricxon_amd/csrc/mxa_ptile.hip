@@ -645,25 +645,31 @@ int launch_moe_p_type(const uint8_t* w, long long row_bytes, long long expert_st
 int launch_moe_ptile(int type, const uint8_t* w, long long row_bytes, long long expert_stride, int n_experts,
                      const Act& act, const int32_t* offsets, int total_rows, YOut y, long long ldy, int n_rows,
                      hipStream_t stream) {
-  auto go = [&](auto f) {
-    return f(w, row_bytes, expert_stride, n_experts, act, offsets, total_rows, y, ldy, n_rows, stream);
-  };
-  switch (type) {
-    case T_Q4_K: return go(launch_moe_p_type<T_Q4_K>);
-    case T_Q6_K: return go(launch_moe_p_type<T_Q6_K>);
-    case T_Q8_0: return go(launch_moe_p_type<T_Q8_0>);
-    default: return -1;
+  const int step = prow_limit(row_bytes);
+  for (long long n0 = 0; n0 < n_rows; n0 += step) {
+    auto go = [&](auto f) {
+      return f(w + n0 * row_bytes, row_bytes, expert_stride, n_experts, act, offsets, total_rows, y.at(n0), ldy,
+               (int)min((long long)step, n_rows - n0), stream);
+    };
+    const int st = type == T_Q4_K ? go(launch_moe_p_type<T_Q4_K>) : type == T_Q6_K ? go(launch_moe_p_type<T_Q6_K>)
+                 : type == T_Q8_0 ? go(launch_moe_p_type<T_Q8_0>) : -1;
+    if (st != 0) return st;
   }
+  return 0;
 }
 
 int launch_ptile(int type, const uint8_t* w, long long row_bytes, const Act& act, YOut y, long long ldy,
                  int m_rows, int n_rows, hipStream_t stream) {
-  switch (type) {
-    case T_Q4_K: return launch_p_type<T_Q4_K>(w, row_bytes, act, y, ldy, m_rows, n_rows, stream);
-    case T_Q6_K: return launch_p_type<T_Q6_K>(w, row_bytes, act, y, ldy, m_rows, n_rows, stream);
-    case T_Q8_0: return launch_p_type<T_Q8_0>(w, row_bytes, act, y, ldy, m_rows, n_rows, stream);
-    default: return -1;
+  const int step = prow_limit(row_bytes);
+  for (long long n0 = 0; n0 < n_rows; n0 += step) {
+    auto go = [&](auto f) {
+      return f(w + n0 * row_bytes, row_bytes, act, y.at(n0), ldy, m_rows, (int)min((long long)step, n_rows - n0), stream);
+    };
+    const int st = type == T_Q4_K ? go(launch_p_type<T_Q4_K>) : type == T_Q6_K ? go(launch_p_type<T_Q6_K>)
+                 : type == T_Q8_0 ? go(launch_p_type<T_Q8_0>) : -1;
+    if (st != 0) return st;
   }
+  return 0;
 }
 
 }  // namespace mxa

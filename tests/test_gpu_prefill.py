@@ -134,3 +134,22 @@ def test_grouped_prefill_expert_strides(gpu, oracle, t) -> None:
         if c:
             rows = slice(off[i], off[i + 1])
             assert np.array_equal(bits(got[rows]), bits(oracle.gemm(t, w[i], x[rows], n, k)))
+
+
+@pytest.mark.parametrize("t", [D.Q8_0, D.IQ4_XS])
+def test_prefill_rows_past_4_gib_apart(gpu, t) -> None:
+    """Rows so long that a wave's last ones start more than 4 GiB past its first: they equal the same rows of
+    a matrix of two, of which neither does."""
+    k = 256 * (540_000 if t == D.Q8_0 else 1_080_000)
+    rb, n, m = gpu.row_bytes(t, k), 32, 17
+    assert 30 * rb > 1 << 32
+    g = torch.Generator(device="cuda").manual_seed(5)
+    w = torch.randint(0, 256, (n, rb), dtype=torch.uint8, device="cuda", generator=g)
+    blocks = w.view(-1, 34 if t == D.Q8_0 else 136)
+    blocks[:, 0] = torch.randint(0, 256, (blocks.shape[0],), dtype=torch.uint8, device="cuda", generator=g)
+    blocks[:, 1] = 0x0C  # scales of 2^-12 to 2^-11
+    x = torch.randn((m, k), device="cuda", generator=g)
+    got = gpu.matmul(t, w, x, n, k)
+    for r in (0, 30) if t == D.Q8_0 else (30,):
+        assert torch.equal(got[:, r:r + 2].view(torch.int32), gpu.matmul(t, w[r:r + 2], x, 2, k).view(torch.int32))
+    assert got.isfinite().all() and got[:, 31].count_nonzero() == m
