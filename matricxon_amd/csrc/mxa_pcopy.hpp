@@ -28,6 +28,8 @@ inline int prow_limit(long long row_bytes) {
   const long long rows = ((1LL << 32) - 512) / row_bytes;
   return rows >= 32 ? 0x7FFFFFFF : rows > 1 ? (int)rows : 1;
 }
+// Activation rows that one launch takes: 65535 groups of 64 in the grid's second dimension.
+constexpr int kMaxPrefillRows = 65535 * 64;
 
 // A wave's 32 weight rows, copied block by block into a slot that only it reads. Piece c of row q comes
 // from the 16-byte boundary at or below the block's start. Every piece holds at least one byte of the

@@ -661,14 +661,20 @@ int launch_moe_ptile(int type, const uint8_t* w, long long row_bytes, long long 
 int launch_ptile(int type, const uint8_t* w, long long row_bytes, const Act& act, YOut y, long long ldy,
                  int m_rows, int n_rows, hipStream_t stream) {
   const int step = prow_limit(row_bytes);
-  for (long long n0 = 0; n0 < n_rows; n0 += step) {
-    auto go = [&](auto f) {
-      return f(w + n0 * row_bytes, row_bytes, act, y.at(n0), ldy, m_rows, (int)min((long long)step, n_rows - n0), stream);
-    };
-    const int st = type == T_Q4_K ? go(launch_p_type<T_Q4_K>) : type == T_Q6_K ? go(launch_p_type<T_Q6_K>)
-                 : type == T_Q8_0 ? go(launch_p_type<T_Q8_0>) : -1;
-    if (st != 0) return st;
-  }
+  for (long long m0 = 0; m0 < m_rows; m0 += kMaxPrefillRows)
+    for (long long n0 = 0; n0 < n_rows; n0 += step) {
+      Act a = act;
+      a.q = act.q + m0 * act.k;
+      a.d = act.d + m0 * act.nb;
+      a.bsums = act.bsums + m0 * act.nb * 16;
+      auto go = [&](auto f) {
+        return f(w + n0 * row_bytes, row_bytes, a, y.at(m0 * ldy + n0), ldy,
+                 (int)min((long long)kMaxPrefillRows, m_rows - m0), (int)min((long long)step, n_rows - n0), stream);
+      };
+      const int st = type == T_Q4_K ? go(launch_p_type<T_Q4_K>) : type == T_Q6_K ? go(launch_p_type<T_Q6_K>)
+                   : type == T_Q8_0 ? go(launch_p_type<T_Q8_0>) : -1;
+      if (st != 0) return st;
+    }
   return 0;
 }
 

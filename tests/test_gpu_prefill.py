@@ -153,3 +153,13 @@ def test_prefill_rows_past_4_gib_apart(gpu, t) -> None:
     for r in (0, 30) if t == D.Q8_0 else (30,):
         assert torch.equal(got[:, r:r + 2].view(torch.int32), gpu.matmul(t, w[r:r + 2], x, 2, k).view(torch.int32))
     assert got.isfinite().all() and got[:, 31].count_nonzero() == m
+
+
+def test_prefill_more_rows_than_a_grid_takes(gpu, oracle) -> None:
+    """More than 65535 groups of 64 activation rows, the most of one launch's grid."""
+    n, k, m = 3, 256, 65535 * 64 + 70
+    w = S.packed_weight(D.Q4_K, n, k, seed=2)
+    x = torch.randn((m, k), device="cuda", generator=torch.Generator(device="cuda").manual_seed(6))
+    got = gpu.matmul(D.Q4_K, dev(w), x, n, k)
+    for rows in (slice(0, 40), slice(m - 130, m)):
+        assert np.array_equal(bits(host(got[rows])), bits(oracle.gemm(D.Q4_K, w, host(x[rows]), n, k)))
