@@ -49,11 +49,12 @@ def test_prefill_weight_alignment(gpu, oracle, t, shift, m) -> None:
     check(gpu, oracle, t, w, S.activations(m, 1280, seed=10), n, 1280, shift)
 
 
-@pytest.mark.parametrize("t", TYPES)
+@pytest.mark.parametrize("t,q6_scale", [(D.Q4_K, 0), (D.Q6_K, -128), (D.Q6_K, -4), (D.Q8_0, 0)])
 @pytest.mark.parametrize("sign", [1, -1])
-def test_prefill_largest_sums(gpu, oracle, t, sign) -> None:
+def test_prefill_largest_sums(gpu, oracle, t, q6_scale, sign) -> None:
     """Every code, scale and activation at its largest magnitude, all products of one sign: the sums
-    that the float conversion of the integer planes has to hold."""
+    that the float conversion of the integer planes has to hold. Q6_K's value -32 times a scale of -128 is
+    16 in the high plane and 0 in the low one, times -4 it is 1 and -128, that plane's largest."""
     n, k, m = 40, 1536, 80
     w = S.packed_weight(t, n, k, seed=1).reshape(n, -1)
     if t == D.Q4_K:
@@ -63,7 +64,7 @@ def test_prefill_largest_sums(gpu, oracle, t, sign) -> None:
     elif t == D.Q6_K:
         b = w.reshape(-1, 210)
         b[:, :192] = 0  # every code 0, the value -32
-        b[:, 192:208] = 0x80  # every scale -128
+        b[:, 192:208] = q6_scale & 0xFF
     else:
         w.reshape(-1, 34)[:, 2:] = 0x80  # every quant -128
     x = np.full((m, k), 127.0 * sign, dtype=np.float32)
@@ -163,3 +164,15 @@ def test_prefill_more_rows_than_a_grid_takes(gpu, oracle) -> None:
     got = gpu.matmul(D.Q4_K, dev(w), x, n, k)
     for rows in (slice(0, 40), slice(m - 130, m)):
         assert np.array_equal(bits(host(got[rows])), bits(oracle.gemm(D.Q4_K, w, host(x[rows]), n, k)))
+
+
+@pytest.mark.parametrize("t", TYPES)
+@pytest.mark.parametrize("m", [4, 9, 16])
+@pytest.mark.parametrize("shift", [0, 4])
+def test_wide_matrices_of_few_rows(gpu, oracle, t, m, shift) -> None:
+    """4 to 16 activation rows and 32768 weight rows or more, also where the weights' place or the length of a
+    row keeps the batched-decode kernels from taking them."""
+    n, k = 32800, 256 * 18
+    w = S.packed_weight(t, 64, k, seed=3)
+    w = np.ascontiguousarray(np.tile(w, (n // 64 + 1, 1))[:n])
+    check(gpu, oracle, t, w, S.activations(m, k, seed=m), n, k, shift)

@@ -102,3 +102,11 @@ def test_finish_gives_the_leading_shape() -> None:
     for lead in ((5,), (12,), (2, 2)):
         with pytest.raises(RuntimeError):
             mod.finish(torch.zeros(6, N), lead)
+
+
+def test_supports_is_the_librarys_rule() -> None:
+    """`HipGemm.supports` answers the common case itself; every answer is the library's."""
+    gemm = HipGemm.get()
+    for t in range(-1, 40):
+        for k in (-256, 0, 1, 32, 255, 256, 288, 512, 2816, 4096, 4097, (1 << 31) - 256):
+            assert gemm.supports(t, k) == bool(gemm._lib.mxa_supports(t, k)), (t, k)
