@@ -156,11 +156,11 @@ class DevicePackedLinear(nn.Module):
         return self._dtype
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        lead = x.shape[:-1]
-        k = self.in_features
+        shape, k = x.shape, self.in_features
+        lead = shape[:-1]
         # As F.linear: the rows are passed by address below, so nothing after this compares widths.
-        if x.shape[-1:] != (k,) and x.numel() > 0:
-            raise RuntimeError(f"x must have {k} values in its last dimension, got shape {tuple(x.shape)}")
+        if (not shape or shape[-1] != k) and x.numel() > 0:
+            raise RuntimeError(f"x must have {k} values in its last dimension, got shape {tuple(shape)}")
         if self.backend == "numba":
             return self.finish(self._forward_f32(x.reshape(-1, k)), lead)
         # The reference casts x to the layer dtype before its matmul (device_packed.py:54).
@@ -169,13 +169,14 @@ class DevicePackedLinear(nn.Module):
         bf16 = self._dtype == torch.bfloat16  # the kernels read and write bfloat16 themselves
         packed = self.packed
         dev = packed.device
-        n, big_n = x.numel() // k, self.out_features
+        rows = len(lead) == 1
+        n, big_n = lead[0] if rows else x.numel() // k, self.out_features
         ws = HANDOFF.claim(x) if self._ggml_type != _IQ4_XS else None
         if ws is not None:  # x came from a fused producer that also wrote its Q8_K blocks
             y = torch.empty((n, big_n), dtype=torch.bfloat16 if bf16 else torch.float32, device=dev)
             self._gemm.matmul_q8k(self._ggml_type, packed, ws, None, y, n, big_n, k)
         elif bf16 and x.device == dev and n > 0:
-            xb = x if x.dim() == 2 else x.reshape(n, k)  # of width k: checked above
+            xb = x if rows else x.reshape(n, k)
             if not xb.is_contiguous() or xb.data_ptr() % 16 != 0:
                 xb = xb.clone(memory_format=torch.contiguous_format)
             y = torch.empty((n, big_n), dtype=torch.bfloat16, device=dev)
