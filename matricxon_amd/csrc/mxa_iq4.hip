@@ -5,7 +5,8 @@
 // parts, x = hi + lo (hi = x rounded to bf16, lo = the rest rounded to bf16; relative error of the
 // pair about 2^-17), written to the workspace by split_bf16_kernel. The grid values are small
 // integers, exact in bf16, so bf16 MFMAs on (hi, K) and (lo, K) give sum(K * x) of one sub-block.
-// The sub-block scale dl is applied in fp32 after them. The result meets the float tolerance against the reference (rel-L2 <= 1e-4); its summation order differs from the
+// The sub-block scale dl is applied in fp32 after them. The result
+// meets the float tolerance against the reference (rel-L2 <= 1e-4); its summation order differs from the
 // decode kernels', which is why batches of up to 16 rows stay on those.
 #include "mxa_kernels.hpp"
 #include "mxa_pcopy.hpp"
@@ -68,11 +69,13 @@ __device__ __forceinline__ u32x4a4 grid_bf16x8(uint32_t a, uint32_t b) {
 // The activations of half a block (128 values: 256 bytes of hi, 256 of lo per row) go straight into one of
 // two LDS buffers, piece c of row r at place c ^ (r & 15); a wave's weights into a slot that only it reads.
 //
-// Bound: instruction issue (a sub-block of 32 rows costs about 50 VALU instructions to look its 512
-// values up as bf16, 16 per activation tile to scale, four MFMAs of 32 cycles per tile). Measured on
-// MI355X against 16 x 16 tiles whose eight waves read every operand from LDS (us per call, the same bits):
-// 4096 x 4096 M = 512 58 vs 94, M = 2048 200 vs 283 (344 TFLOP/s), 14336 x 4096 M = 2048 632 vs 941,
-// 4096 x 14336 M = 128 129 vs 261.
+// Bound: latency at few waves. A sub-block of 32 rows costs about 50 VALU instructions to look its 512 values
+// up as bf16, and 16 to scale and four MFMAs of 32 cycles per activation tile; at 4096 x 4096 M = 512 one wave
+// stands on a SIMD, whose VALU issues in 43% of the cycles and whose matrix core is busy in 24%, with nothing
+// to run in its waits. At M = 2048 two waves do.
+// Measured on MI355X against 16 x 16 tiles whose eight waves read every operand from LDS (us per call with
+// the split, the same bits): 4096 x 4096 M = 64 41 vs 83, M = 512 58 vs 87, M = 2048 180 vs 282 (382 TFLOP/s),
+// 14336 x 4096 M = 2048 610 vs 944, 4096 x 14336 M = 128 131 vs 248.
 struct PIQ4 {
   static constexpr int kBytes = 136, kShift = 8;  // blocks start at 8-byte multiples of the row
 };
@@ -196,8 +199,8 @@ int launch_iq4_prefill(const uint8_t* w, long long row_bytes, const float* x, vo
     };
     // Two activation tiles share a wave's looked-up weights, and eight waves an activation block in LDS,
     // while the grid fills the chip. Measured on MI355X, us per call with the split, eight waves of two
-    // tiles / four of two / two of one: 4096 x 4096 M = 2048 (512 workgroups of the first form) 200 / 215 /
-    // 326, M = 512 (128) 86 / 58 / 93, M = 64 (16) 79 / 52 / 40; 14336 x 4096 M = 512 (448) 169 / 203 / 273.
+    // tiles / four of two / two of one: 4096 x 4096 M = 2048 (512 workgroups of the first form) 183 / 216 /
+    // 317, M = 512 (128) 83 / 58 / 92, M = 64 (16) 80 / 53 / 41; 14336 x 4096 M = 512 (448) 166 / 200 / 269.
     const long long m_tiles = (m_rows + 63) / 64, cus = cu_count();
     if ((n_rows + 255) / 256 * m_tiles >= cus) go(iq4_ptile_kernel<8, 2>, 8, 2);
     else if ((n_rows + 127) / 128 * m_tiles >= cus * 3 / 4) go(iq4_ptile_kernel<4, 2>, 4, 2);

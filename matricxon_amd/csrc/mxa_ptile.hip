@@ -18,13 +18,20 @@
 // slot that only it reads: it takes the block into registers and refills the slot at once. Loading
 // the weights per lane into registers instead cost a fifth (Q4_K) to a half (Q6_K) of the time.
 //
-// Bound: instruction issue. Per 32 x 64 x 256 step a Q4_K wave issues 340 VALU instructions (80 a tile
-// to fold, 150 to decode, the rest addresses) and 34 MFMAs of 32 cycles; two waves share a SIMD, the
-// matrix cores are busy 39% of the time, and more stages of copies ahead or another order of the
-// instructions change nothing. Measured on MI355X against the 16 x 16 tiles before (us, kernel alone):
-// Q4_K 14336 x 4096 M = 2048 320 vs 376 (750 TFLOP/s equivalent), Q6_K 4096 x 14336 M = 1024 239 vs 494
-// (its sub-block scales went into two planes: 16 quarter-filled MFMAs and 64 integer products per
-// output quad before), Q8_0 4096 x 4096 M = 2048 111 vs 247, M = 333 36 vs 58.
+// Bound: no unit of its own. A 32 x 64 x 256 step of a Q4_K wave issues about 430 VALU instructions (decode,
+// fold, addresses) and 34 MFMAs of 32 cycles. Over Q4_K 14336 x 4096 M = 2048 VALU instructions issue in 56%
+// of a SIMD's cycles and the matrix cores are busy in 33%, of which 59% beside VALU instructions; the waves
+// spend 31% of their time in waits. Q6_K 4096 x 14336 M = 1024: 52%, 19%, 56%, and 25%; 29% goes to waiting to
+// issue LDS reads (12% for Q4_K), which start at 2-byte places and lose 12 cycles each to bank conflicts (3.5).
+// Two waves share a SIMD and meet at every block's barrier, so decode, MFMAs and folds overlap in part only;
+// more stages of copies ahead or another order of the instructions change nothing.
+//
+// Measured on MI355X against the 16 x 16 tiles before (us, kernel alone, weights from HBM): Q4_K 14336 x 4096
+// M = 2048 321 vs 351 (750 TFLOP/s equivalent), M = 512 88 vs 96, M = 64 24 vs 52; Q6_K 4096 x 14336 M = 1024 246
+// vs 488 (its sub-block scales went into two planes: 16 quarter-filled MFMAs and 64 integer products per
+// output quad before), 128256 x 4096 M = 32 159 vs 414; Q8_0 4096 x 4096 M = 2048 113 vs 258, M = 333 37 vs 58.
+// Q4_K weights that start off a 16-byte boundary lose 5 to 17% to them: their blocks are read from LDS at
+// dword places.
 //
 // Numerics: integer sums are exact and the fp32 steps are the oracle's, in block order, so the
 // outputs equal the decode kernels' bit for bit.
@@ -481,9 +488,10 @@ __global__ __launch_bounds__(64 * WN, 2) void moe_ptile_kernel(const uint8_t* w,
 // its own copies of both operands. A round's block values meet in LDS, and wave j folds the outputs of
 // activation rows 8 j .. 8 j + 7 of each half, blocks in order, so the bits are the same.
 //
-// Bound: a wave alone on its SIMD takes about 1.1 us a block (one instruction per ~6 cycles, the copies'
-// latency), so what counts is the number of blocks in a row that one wave takes and the waves in
-// flight: two workgroups fit a CU (74 KB of LDS for Q4_K).
+// Bound: latency. A workgroup alone on its CU takes 1.8 us a round of four blocks (Q4_K; Q6_K 2.8, Q8_0 2.3):
+// the wait for its copies, a decode and MFMAs that no other wave of the SIMD covers, two barriers. So what
+// counts is the number of rounds and the waves in flight: two workgroups fit a CU (74 KB of LDS for Q4_K, 78
+// for Q6_K; Q8_0's 86 leave one).
 constexpr int kKs = 4;
 template <class T>
 constexpr int ks_act_bytes() { return 32 * QK + (T::kBsums ? 1024 : 0) + 256; }
@@ -593,14 +601,15 @@ int launch_p(const uint8_t* w, long long row_bytes, const Act& act, YOut y, long
 
 // Few 32 x 32 tiles take a workgroup each. Otherwise two activation tiles share a wave's decoded
 // weights, and eight waves an activation block in LDS, as long as the grid still fills the chip.
-// Measured on MI355X, us, kernel alone; workgroup per tile / two waves of one tile / four of two:
-//   Q4_K 4096 x 4096 M = 32 / 128 / 200 / 333 (128 / 512 / 896 / 1408 tiles) 9.8 / 20 / 28, 12.6 / 20 / 28,
-//   21 / 28 / 29, 31 / 34 / 30; 14336 x 4096 M = 64 / 128 (896 / 1792) 23 / 29 / 29, 40 / 34 / 30; Q6_K
-//   4096 x 14336 M = 256 (1024) 117 / 165 / -; Q8_0 4096 x 4096 M = 128 / 333 (512 / 1408) 23 / 27 / 43,
-//   62 / 36 / 45, 14336 x 4096 M = 48 (896; its workgroup per tile has a CU to itself) 49 / 32 / -;
-// eight waves of two tiles / four of two / two of one: Q4_K 14336 x 4096 M = 2048 326 / 336 / 446, 4096 x
-//   4096 M = 1024 46.0 / 47.7 / 69; Q6_K 4096 x 14336 M = 1024 239 / 247 / 443; Q8_0 4096 x 4096 M = 2048
-//   114 / 111 / 157.
+// Measured on MI355X, us, kernel alone, weights from HBM; workgroup per tile / two waves of one tile / four of two:
+//   Q4_K 4096 x 4096 M = 32 / 128 / 200 / 333 (128 / 512 / 896 / 1408 tiles) 11 / 21 / 29, 13 / 21 / 30,
+//   23 / 30 / 30, 32 / 31 / 30; 14336 x 4096 M = 64 / 128 (896 / 1792) 24 / 29 / 30, 40 / 35 / 31; Q6_K
+//   4096 x 14336 M = 256 (1024) 124 / 172 / 152; Q8_0 4096 x 4096 M = 128 / 333 (512 / 1408) 24 / 30 / 45,
+//   62 / 37 / 46, 14336 x 4096 M = 48 (896; its workgroup per tile has a CU to itself) 49 / 34 / 46;
+// eight waves of two tiles / four of two / two of one: Q4_K 14336 x 4096 M = 2048 321 / 303 / 427, 4096 x
+//   4096 M = 1024 48 / 49 / 70, 128256 x 4096 M = 32 106 / 101 / 94 (half of every second tile's rows are
+//   repeats); Q6_K 4096 x 14336 M = 1024 250 / 250 / 453, 128256 x 4096 M = 32 159 / 156 / 144; Q8_0 4096 x 4096
+//   M = 2048 116 / 112 / 158.
 template <int TYPE>
 int launch_p_type(const uint8_t* w, long long row_bytes, const Act& act, YOut y, long long ldy, int M, int N,
                   hipStream_t stream) {
@@ -632,9 +641,12 @@ int launch_moe_p(const uint8_t* w, long long row_bytes, long long expert_stride,
 template <int TYPE>
 int launch_moe_p_type(const uint8_t* w, long long row_bytes, long long expert_stride, int n_experts, const Act& act,
                       const int32_t* offsets, int total_rows, YOut y, long long ldy, int N, hipStream_t stream) {
-  // 64-row chunks once an expert has more than 32 rows on average (MI355X, us, 64- / 32-row chunks:
-  // 64 experts top 8, 512 tokens, Q6_K 2048 x 1024 63 / 78, Q4_K 1024 x 2048 49 / 45; 8 experts top 2
-  // at 256 tokens, Q4_K 14336 x 4096 129 / 150, at 96 tokens 69 / 65)
+  // 64-row chunks once an expert has more than 32 rows on average: fewer workgroups read its weights.
+  // Measured on MI355X, us, 64- / 32-row chunks, random routings: 8 experts, Q4_K 14336 x 4096 28 / 33 / 48 / 96
+  // rows an expert 81 / 82, 91 / 97, 104 / 119, 169 / 193, Q6_K 4096 x 14336 22 / 33 / 64 rows 142 / 142, 158 / 225,
+  // 249 / 307; over ten expert sets past 32 rows 64-row chunks take 0.92 (Q4_K), 0.78 (Q6_K) and
+  // 0.85 (Q8_0) of the time on average, but up to 1.3 where few rows of few experts leave half the chip idle
+  // (8 experts, Q4_K 2048 x 8192 33 to 56 rows 57 / 47).
   if (total_rows > 32LL * n_experts)
     return launch_moe_p<TYPE, 4, 2>(w, row_bytes, expert_stride, n_experts, act, offsets, total_rows, y, ldy, N, stream);
   return launch_moe_p<TYPE, 4, 1>(w, row_bytes, expert_stride, n_experts, act, offsets, total_rows, y, ldy, N, stream);
