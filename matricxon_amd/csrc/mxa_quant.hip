@@ -85,10 +85,11 @@ void launch_widen_bf16(const uint16_t* x, float* out, long long n, hipStream_t s
 // An embedding lookup is launch-bound, so it is one launch: int64 ids wrapped here and bfloat16 written
 // here (512 ids of Q6_K 128256 x 4096 took 47 us in six launches, 11 now, all of it the host's call).
 
+// The source is known to the compiler (Id: char for a flat array, int32_t for rows, int64_t for ids, the one
+// that may write bfloat16): chosen in the kernel, it cost row gathers 3%.
 struct DequantSrc {
   const uint8_t* base;
-  const int32_t* rows;  // null: flat block array (unless ids is given)
-  const int64_t* ids;   // token ids in place of rows: a negative one counts from the end, once
+  const void* rows;  // int32 rows, or int64 token ids: a negative one counts from the end, once
   long long n_src_rows;
   long long row_bytes;
   int blocks_per_row;
@@ -187,8 +188,9 @@ __device__ __forceinline__ void dequant8<T_IQ4_XS>(const uint8_t* __restrict__ b
   }
 }
 
-template <int TYPE>
+template <int TYPE, class Id>
 __global__ __launch_bounds__(256) void dequant_kernel(DequantSrc src, long long n_blocks, YOut out) {
+  constexpr bool kIds = sizeof(Id) == 8;
   constexpr int kThreads = Geo<TYPE>::kElems / 8;
   const long long t = (long long)blockIdx.x * 256 + threadIdx.x;
   const long long g = t / kThreads;
@@ -197,11 +199,11 @@ __global__ __launch_bounds__(256) void dequant_kernel(DequantSrc src, long long 
   float v[8];
   bool ok = true;
   const uint8_t* blk;
-  if (src.rows != nullptr || src.ids != nullptr) {
+  if constexpr (sizeof(Id) > 1) {
     const long long r = g / src.blocks_per_row;
     const long long bi = g - r * src.blocks_per_row;
-    long long row = src.ids != nullptr ? src.ids[r] : src.rows[r];
-    if (src.ids != nullptr && row < 0) row += src.n_src_rows;
+    long long row = ((const Id*)src.rows)[r];
+    if (kIds && row < 0) row += src.n_src_rows;
     ok = row >= 0 && row < src.n_src_rows;
     blk = src.base + (ok ? row : 0) * src.row_bytes + bi * Geo<TYPE>::kBytes;
   } else {
@@ -213,7 +215,7 @@ __global__ __launch_bounds__(256) void dequant_kernel(DequantSrc src, long long 
 #pragma unroll
     for (int i = 0; i < 8; ++i) v[i] = __builtin_nanf("");
   }
-  if (out.is_bf16()) {
+  if (kIds && out.is_bf16()) {
     uint32_t h[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) h[i] = (uint32_t)bf16_rne(v[2 * i]) | ((uint32_t)bf16_rne(v[2 * i + 1]) << 16);
@@ -226,22 +228,23 @@ __global__ __launch_bounds__(256) void dequant_kernel(DequantSrc src, long long 
 }
 
 template <int TYPE>
-static void launch_dequant_t(const DequantSrc& src, long long n_blocks, YOut out, hipStream_t stream) {
+static void launch_dequant_t(const DequantSrc& src, bool ids, long long n_blocks, YOut out, hipStream_t stream) {
   const long long threads = n_blocks * (Geo<TYPE>::kElems / 8);
   const long long grid = (threads + 255) / 256;
-  hipLaunchKernelGGL(dequant_kernel<TYPE>, dim3((unsigned)grid), dim3(256), 0, stream, src,
-                     n_blocks, out);
+  auto kern = src.rows == nullptr ? dequant_kernel<TYPE, char> : ids ? dequant_kernel<TYPE, int64_t> : dequant_kernel<TYPE, int32_t>;
+  hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(256), 0, stream, src, n_blocks, out);
 }
 
 int launch_dequant(int type, const uint8_t* base, const int32_t* rows, const int64_t* ids,
                    long long n_src_rows, long long row_bytes, int blocks_per_row, long long n_blocks,
                    YOut out, hipStream_t stream) {
-  const DequantSrc src{base, rows, ids, n_src_rows, row_bytes, blocks_per_row};
+  const bool by_id = ids != nullptr;
+  const DequantSrc src{base, by_id ? (const void*)ids : rows, n_src_rows, row_bytes, blocks_per_row};
   switch (type) {
-    case T_Q8_0: launch_dequant_t<T_Q8_0>(src, n_blocks, out, stream); return 0;
-    case T_Q4_K: launch_dequant_t<T_Q4_K>(src, n_blocks, out, stream); return 0;
-    case T_Q6_K: launch_dequant_t<T_Q6_K>(src, n_blocks, out, stream); return 0;
-    case T_IQ4_XS: launch_dequant_t<T_IQ4_XS>(src, n_blocks, out, stream); return 0;
+    case T_Q8_0: launch_dequant_t<T_Q8_0>(src, by_id, n_blocks, out, stream); return 0;
+    case T_Q4_K: launch_dequant_t<T_Q4_K>(src, by_id, n_blocks, out, stream); return 0;
+    case T_Q6_K: launch_dequant_t<T_Q6_K>(src, by_id, n_blocks, out, stream); return 0;
+    case T_IQ4_XS: launch_dequant_t<T_IQ4_XS>(src, by_id, n_blocks, out, stream); return 0;
     default: return -1;
   }
 }
